@@ -46,122 +46,300 @@ __global__ void km_init_kernel(const void* x, int dt, int64_t S, int64_t H, int6
   if (d < D) cent[(bh * K + j) * D + d] = load_as_f32(x, ((b * S + idx) * H + h) * D + d, dt);
 }
 
-// n consecutive elements of dtype DT as fp32 (n a multiple of 8, 16-byte aligned)
-template <int DT, int N>
-__device__ __forceinline__ void load_row(const void* x, int64_t idx, float (&v)[N]) {
-  if constexpr (DT == kF32) {
-    const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(x) + idx);
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// 8 consecutive elements of dtype DT: as loaded, and as fp32
+template <int DT>
+struct Raw8 {
+  uint4 r[DT == kF32 ? 2 : 1];
+  __device__ __forceinline__ void load(const void* x, int64_t idx) {
+    const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(x) + idx * (DT == kF32 ? 4 : 2));
+    r[0] = p[0];
+    if constexpr (DT == kF32) r[1] = p[1];
+  }
+  __device__ __forceinline__ void to_f32(float (&v)[8]) const {
+    const uint32_t w[4] = {r[0].x, r[0].y, r[0].z, r[0].w};
+    if constexpr (DT == kF32) {
+      const uint32_t w1[4] = {r[1].x, r[1].y, r[1].z, r[1].w};
 #pragma unroll
-    for (int i = 0; i < N / 4; ++i) {
-      const float4 f = p[i];
-      v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
-    }
-  } else {
-    const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(x) + idx);
-#pragma unroll
-    for (int i = 0; i < N / 8; ++i) {
-      const uint4 r = p[i];
-      const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+      for (int k = 0; k < 4; ++k) { v[k] = __uint_as_float(w[k]); v[4 + k] = __uint_as_float(w1[k]); }
+    } else {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const uint16_t lo = static_cast<uint16_t>(w[k] & 0xffffu), hi = static_cast<uint16_t>(w[k] >> 16);
-        if constexpr (DT == kBF16) { v[8 * i + 2 * k] = bf16_bits_to_f32(lo); v[8 * i + 2 * k + 1] = bf16_bits_to_f32(hi); }
-        else { v[8 * i + 2 * k] = f16_bits_to_f32(lo); v[8 * i + 2 * k + 1] = f16_bits_to_f32(hi); }
+        if constexpr (DT == kBF16) { v[2 * k] = bf16_bits_to_f32(lo); v[2 * k + 1] = bf16_bits_to_f32(hi); }
+        else { v[2 * k] = f16_bits_to_f32(lo); v[2 * k + 1] = f16_bits_to_f32(hi); }
       }
     }
   }
+};
+
+template <int DT>
+__device__ __forceinline__ void load8(const void* x, int64_t idx, float (&v)[8]) {
+  Raw8<DT> r;
+  r.load(x, idx);
+  r.to_f32(v);
 }
 
-// One thread per token: its row in registers (16-byte loads), the slice's
-// centroids in LDS read as float4 broadcasts; each distance is the sequential
-// fmaf chain over d of the specification.
+// v = hi + lo + r with hi = bf16(v), lo = bf16(v - hi), |r| <= 2^-18 |v|
+// (v - hi is exact; both roundings to nearest)
+__device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    hi[i] = static_cast<__bf16>(v[i]);
+    lo[i] = static_cast<__bf16>(v[i] - static_cast<float>(hi[i]));
+  }
+}
+
+// ---- assignment ------------------------------------------------------------------
+// The labels of the specification (first minimum of fmaf(-2, dot_j, cn_j) over
+// sequential fp32 FMA chains), found on the matrix cores and settled exactly
+// where they cannot decide.
+//
+// A wave takes 32 tokens.  v_mfma_f32_32x32x16_bf16 forms
+// a_j = dot_j - cn_j / 2 for 32 centroids at a time (rows: centroids, read as
+// hi / lo bf16 pairs from LDS; columns: tokens, straight from global memory --
+// bf16 tokens are exact, fp16 / fp32 ones are split in hi + lo as well).  The
+// largest a_j belongs to the smallest score.  With X = |x|_2 and
+// C = max_j |c_j|_2 (so sum_d |x_d c_d| <= X C), the errors of a_j are at most
+//   the specification's own chain    2^-17 X C       (128 FMA roundings)
+//   its last rounding                2^-24 (X C + C^2 / 2)
+//   operands split in two            2^-18 X C       (3 * 2^-18 X C when x is split too: the
+//                                                     residuals of both and the lo * lo term)
+//   accumulation                     2^-20 (X C + C^2 / 2) per MFMA: 16, or 24 with x split
+// the last at twice the largest error of an MFMA measured on a gfx950 relative
+// to the magnitudes it adds (2^-21.4 over operands of mixed magnitude, 2^-23
+// over operands of one).  Twice their sum is below 2^-14 X C + 2^-15 C^2
+// (2^-13 and 2^-14 with x split): two centroids whose a_j are further apart
+// than that gap are in the specification's order.  A token with another
+// centroid within the gap of its best -- or with a non-finite value anywhere,
+// since the test counts the centroids that are NOT below the gap -- is settled
+// by the specification itself: one lane per centroid runs the FMA chain, and
+// the wave takes the first minimum.
+//
+// Bound by the token reads: 40 x 32768 x 128 bf16 (335 MB a round) with 32
+// clusters took 196 us as one token per lane against LDS broadcasts (1.7 TB/s;
+// 278 us with 64 clusters: the FMA issue bound it).
+constexpr int kAsgWaves = 8;
+constexpr int kAsgThreads = 64 * kAsgWaves;
+constexpr int kSlab = 32 * kAsgWaves;  // tokens per step of a workgroup
+
+template <int D, int MB>
+struct AssignLds {
+  static constexpr int P = D + 4;  // row pitch of the fp32 centroids: float4 reads of 16 rows hit distinct banks
+  uint4 part[2][D / 16][MB][64];   // hi / lo operands, as the lanes read them
+  float cent[32 * MB * P];
+  float cn[32 * MB];
+};
+
+// The centroids of slice bh into LDS: fp32 rows, hi / lo MFMA operands and the
+// norms (the specification's chain).  Rows K .. 32 MB - 1 are zero with norm
+// +inf, so they never win.
+template <int D, int MB>
+__device__ __forceinline__ void assign_fill(AssignLds<D, MB>& lds, const float* cent, int K) {
+  using L = AssignLds<D, MB>;
+  constexpr int C8 = D / 8;
+  for (int e = threadIdx.x; e < 32 * MB * C8; e += kAsgThreads) {
+    const int j = e / C8, c8 = e % C8;
+    float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (j < K) load8<kF32>(cent, j * D + 8 * c8, v);
+    float4* row = reinterpret_cast<float4*>(lds.cent + j * L::P + 8 * c8);
+    row[0] = make_float4(v[0], v[1], v[2], v[3]);
+    row[1] = make_float4(v[4], v[5], v[6], v[7]);
+    bf16x8 hi, lo;
+    split8(v, hi, lo);
+    lds.part[0][c8 / 2][j / 32][j % 32 + 32 * (c8 & 1)] = __builtin_bit_cast(uint4, hi);
+    lds.part[1][c8 / 2][j / 32][j % 32 + 32 * (c8 & 1)] = __builtin_bit_cast(uint4, lo);
+  }
+  __syncthreads();
+  if (threadIdx.x < 32 * MB) {
+    const float4* c = reinterpret_cast<const float4*>(lds.cent + threadIdx.x * L::P);
+    float acc = 0.0f;
+#pragma unroll 8
+    for (int i = 0; i < D / 4; ++i) {
+      const float4 v = c[i];
+      acc = fmaf(v.x, v.x, acc);
+      acc = fmaf(v.y, v.y, acc);
+      acc = fmaf(v.z, v.z, acc);
+      acc = fmaf(v.w, v.w, acc);
+    }
+    lds.cn[threadIdx.x] = static_cast<int>(threadIdx.x) < K ? acc : INFINITY;
+  }
+  __syncthreads();
+}
+
+// The specification for one token (its row at element x0) per PER lanes: lane
+// j of the group runs centroid j's chain; returns the label in every lane of
+// the group.  A NaN score never wins, and if nothing does the label is 0.
+template <int D, int DT, int MB>
+__device__ __forceinline__ int assign_exact(const AssignLds<D, MB>& lds, const void* x, int64_t x0, int lane) {
+  constexpr int PER = 32 * MB;
+  const int j = lane % PER;
+  const float* c = lds.cent + j * AssignLds<D, MB>::P;
+  float dot = 0.0f;
+#pragma unroll 4
+  for (int d = 0; d < D; d += 8) {
+    float xv[8];
+    load8<DT>(x, x0 + d, xv);
+    const float4 c0 = *reinterpret_cast<const float4*>(c + d), c1 = *reinterpret_cast<const float4*>(c + d + 4);
+    dot = fmaf(xv[0], c0.x, dot);
+    dot = fmaf(xv[1], c0.y, dot);
+    dot = fmaf(xv[2], c0.z, dot);
+    dot = fmaf(xv[3], c0.w, dot);
+    dot = fmaf(xv[4], c1.x, dot);
+    dot = fmaf(xv[5], c1.y, dot);
+    dot = fmaf(xv[6], c1.z, dot);
+    dot = fmaf(xv[7], c1.w, dot);
+  }
+  float sc = fmaf(-2.0f, dot, lds.cn[j]);
+  int best = j;
+  if (!(sc < INFINITY)) { sc = INFINITY; best = 0; }
+#pragma unroll
+  for (int m = 1; m < PER; m <<= 1) {
+    const float so = __shfl_xor(sc, m, 64);
+    const int bo = __shfl_xor(best, m, 64);
+    if (so < sc || (so == sc && bo < best)) { sc = so; best = bo; }
+  }
+  return best;
+}
+
+// Grid: any number of workgroups; each takes a contiguous share of the
+// BH * ceil(S / kSlab) slabs (two workgroups per CU and equal shares: no
+// partial last wave of workgroups), refilling LDS when the slice changes.
 // prev_changed: the flags of the previous round (NULL in the first round);
 // changed: this round's flags, set to 1 for a slice in which some label
 // changed.  They are zero on entry from the second round on; in the first
 // round every label counts as changed, so every slice's flag is written.
-template <int D, int DT>
-__global__ void __launch_bounds__(256) km_assign_kernel(const void* x, int64_t S, int64_t H, int K, const float* cent,
-                                                        int32_t* labels, const int32_t* prev_changed,
-                                                        int32_t* changed) {
-  __shared__ float4 c_lds[kMaxKAssign * D / 4];
-  __shared__ float cn_lds[kMaxKAssign];
-  const int64_t nblk_s = (S + 255) / 256;
-  const int64_t bh = blockIdx.x / nblk_s;
-  if (prev_changed && prev_changed[bh] == 0) return;  // converged slice (uniform per workgroup)
-  const int64_t t = (blockIdx.x % nblk_s) * 256 + threadIdx.x;
-  const int64_t b = bh / H, h = bh % H;
-  const float4* cg = reinterpret_cast<const float4*>(cent + bh * K * D);
-  for (int i = threadIdx.x; i < K * D / 4; i += 256) c_lds[i] = cg[i];
-  __syncthreads();
-  if (threadIdx.x < K) {
-    const float* c = reinterpret_cast<const float*>(c_lds) + threadIdx.x * D;
-    float acc = 0.0f;
-    for (int d = 0; d < D; ++d) acc = fmaf(c[d], c[d], acc);
-    cn_lds[threadIdx.x] = acc;
-  }
-  __syncthreads();
-  if (t >= S) return;
-  float xv[D];
-  load_row<DT>(x, ((b * S + t) * H + h) * D, xv);
-  float best = INFINITY;
-  int bj = 0;
-  // two centroids at a time: independent dot-product chains (each still
-  // sequential in d), compared in centroid order, so the first minimum wins
-  constexpr int KJ = 2;
-  int j = 0;
-  for (; j + KJ <= K; j += KJ) {
-    float dot[KJ];
+template <int D, int DT, int MB>
+__global__ void __launch_bounds__(kAsgThreads, 4)
+    km_assign_kernel(const void* x, int64_t BH, int64_t S, int64_t H, int K, const float* cent, int32_t* labels,
+                     const int32_t* prev_changed, int32_t* changed) {
+  constexpr int NKS = D / 16;
+  constexpr bool XSPLIT = DT != kBF16;
+  constexpr float kGapXC = XSPLIT ? 0x1p-13f : 0x1p-14f, kGapCC = XSPLIT ? 0x1p-14f : 0x1p-15f;
+  __shared__ AssignLds<D, MB> lds;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = lane & 31, g = lane >> 5;
+  const int64_t nslab = (S + kSlab - 1) / kSlab, total = BH * nslab;
+  const int64_t w0 = total * blockIdx.x / gridDim.x, w1 = total * (blockIdx.x + 1) / gridDim.x;
+  int64_t cur = -1;
+  float c2max = 0.0f;  // >= max_j |c_j|^2
+  for (int64_t w = w0; w < w1; ++w) {
+    const int64_t bh = w / nslab;
+    if (prev_changed && prev_changed[bh] == 0) continue;  // converged slice (uniform per workgroup)
+    if (bh != cur) {
+      if (cur >= 0) __syncthreads();  // every wave is done with the previous slice's centroids
+      assign_fill<D, MB>(lds, cent + bh * K * D, K);
+      cur = bh;
+      c2max = 0.0f;
+      for (int j = 0; j < K; ++j) c2max = fmaxf(c2max, lds.cn[j]);
+      for (int j = 0; j < K; ++j) c2max = lds.cn[j] < INFINITY ? c2max : INFINITY;
+    }
+    const int64_t t0 = (w - bh * nslab) * kSlab + wave * 32;
+    if (t0 >= S) continue;  // no barrier below
+    const int64_t b = bh / H, h = bh - b * H;
+    const int64_t t = t0 + li < S ? t0 + li : S - 1;  // lanes past the end repeat the last token
+    const int64_t x0 = ((b * S + t) * H + h) * D;
+    float xx = 0.0f;
+    v16f a[MB];
 #pragma unroll
-    for (int u = 0; u < KJ; ++u) dot[u] = 0.0f;
+    for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int d4 = 0; d4 < D / 4; ++d4) {
+      for (int r = 0; r < 16; ++r) a[m][r] = -0.5f * lds.cn[32 * m + 8 * (r >> 2) + 4 * g + (r & 3)];
+    // token operands: lane (li, g) holds dimensions 16 ks + 8 g + [0, 8) of its
+    // token, GK k-steps' loads in flight (all; half with fp32 tokens and 64
+    // centroids, to stay under 128 registers)
+    constexpr int GK = DT == kF32 && MB == 2 && NKS == 8 ? 4 : NKS;
+#pragma unroll 1
+    for (int k0 = 0; k0 < NKS; k0 += GK) {
+      Raw8<DT> raw[GK];
 #pragma unroll
-      for (int u = 0; u < KJ; ++u) {
-        const float4 cv = c_lds[(j + u) * (D / 4) + d4];
-        dot[u] = fmaf(xv[4 * d4], cv.x, dot[u]);
-        dot[u] = fmaf(xv[4 * d4 + 1], cv.y, dot[u]);
-        dot[u] = fmaf(xv[4 * d4 + 2], cv.z, dot[u]);
-        dot[u] = fmaf(xv[4 * d4 + 3], cv.w, dot[u]);
+      for (int i = 0; i < GK; ++i) raw[i].load(x, x0 + 16 * (k0 + i) + 8 * g);
+#pragma unroll
+      for (int i = 0; i < GK; ++i) {
+        const int ks = k0 + i;
+        float v[8];
+        raw[i].to_f32(v);
+        bf16x8 xh, xl;
+        split8(v, xh, xl);  // of bf16 tokens xl is zero, and unused
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xx = fmaf(v[e], v[e], xx);
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+          const bf16x8 ch = __builtin_bit_cast(bf16x8, lds.part[0][ks][m][lane]);
+          const bf16x8 cl = __builtin_bit_cast(bf16x8, lds.part[1][ks][m][lane]);
+          a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xh, a[m], 0, 0, 0);
+          a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, xh, a[m], 0, 0, 0);
+          if constexpr (XSPLIT) a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xl, a[m], 0, 0, 0);
+        }
       }
     }
+    xx += __shfl_xor(xx, 32, 64);
+    // X C and C^2 from above: 2^-110 covers squares lost to underflow, 1.001 the roundings of the norms
+    const float xc = sqrtf((xx + 0x1p-110f) * (c2max + 0x1p-110f));
+    const float gap = 1.001f * (kGapXC * xc + kGapCC * c2max) + 0x1p-120f;
+    float top = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < KJ; ++u) {
-      const float sc = fmaf(-2.0f, dot[u], cn_lds[j + u]);
-      if (sc < best) { best = sc; bj = j + u; }
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) top = fmaxf(top, a[m][r]);
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float thr = top - gap;
+    int cnt = 0, bj = 0;
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const bool near = !(a[m][r] < thr);  // NaN on either side counts as near
+        cnt += near ? 1 : 0;
+        bj = near ? 32 * m + 8 * (r >> 2) + (r & 3) : bj;
+      }
+    bj = cnt ? bj + 4 * g : 0;
+    const int cnt2 = cnt + __shfl_xor(cnt, 32, 64);
+    bj = max(bj, __shfl_xor(bj, 32, 64));  // the one near centroid, if there is one
+    // unsettled tokens, two at a time with up to 32 centroids
+    uint32_t open = static_cast<uint32_t>(__ballot(cnt2 != 1 && t0 + li < S));
+    while (open) {
+      const int i0 = __builtin_ctz(open);
+      open &= open - 1;
+      int i1 = i0;
+      if (MB == 1 && open) {
+        i1 = __builtin_ctz(open);
+        open &= open - 1;
+      }
+      const int ti = MB == 1 && lane >= 32 ? i1 : i0;
+      const int lab = assign_exact<D, DT, MB>(lds, x, ((b * S + t0 + ti) * H + h) * D, lane);
+      const int l0 = __builtin_amdgcn_readlane(lab, 0), l1 = __builtin_amdgcn_readlane(lab, 32);
+      if (li == i0) bj = l0;
+      else if (li == i1) bj = l1;
+    }
+    if (lane < 32 && t0 + li < S) {
+      int32_t* lp = labels + bh * S + t0 + li;
+      const int32_t old = prev_changed ? *lp : -1;
+      *lp = bj;
+      if (__any(old != bj) && lane == 0) changed[bh] = 1;
     }
   }
-  for (; j < K; ++j) {
-    const float4* c = c_lds + j * (D / 4);
-    float dot = 0.0f;
-#pragma unroll
-    for (int d4 = 0; d4 < D / 4; ++d4) {
-      const float4 cv = c[d4];
-      dot = fmaf(xv[4 * d4], cv.x, dot);
-      dot = fmaf(xv[4 * d4 + 1], cv.y, dot);
-      dot = fmaf(xv[4 * d4 + 2], cv.z, dot);
-      dot = fmaf(xv[4 * d4 + 3], cv.w, dot);
-    }
-    const float sc = fmaf(-2.0f, dot, cn_lds[j]);
-    if (sc < best) { best = sc; bj = j; }
-  }
-  const int32_t old = prev_changed ? labels[bh * S + t] : -1;
-  labels[bh * S + t] = bj;
-  if (__any(old != bj) && (threadIdx.x & 63) == 0) changed[bh] = 1;
 }
 
 // fp64 per-cluster column sums of one kChunk-token chunk.  The chunk's tokens
 // are first sorted by label in LDS, stably (ballot ranks within a wave, waves
 // and rounds in token order), so a cluster's tokens keep their order.  Then
-// thread (g, d) -- column d, cluster group g -- adds the runs of clusters
-// j = g, g + NG, ... in that order: the token-order fp64 sums of the
-// specification, over chains NG times shorter, with 8 loads in flight.
+// the D / 8 lanes of group g -- 8 columns each, one 16-byte load per bf16 row --
+// add the runs of clusters j = g, g + NG, ... in that order: the token-order
+// fp64 sums of the specification, with 8 rows in flight per lane.
+// Bound by the row reads (and the LDS sort ahead of them); with one column and
+// a 2-byte load per lane it took 132 us a round at 40 x 32768 x 128 bf16, 32
+// clusters (2.5 TB/s).
 constexpr int kUpdThreads = 512;
 
 template <int D, int DT>
 __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const void* x, int64_t S, int64_t H, int K,
                                                                         const int32_t* labels, double* partial,
                                                                         int32_t* counts, const int32_t* changed) {
-  constexpr int NG = kUpdThreads / D;  // cluster groups
+  constexpr int LPG = D / 8;              // lanes per cluster group
+  constexpr int NG = kUpdThreads / LPG;  // cluster groups
   constexpr int NW = kUpdThreads / 64;
   __shared__ int lab_s[kChunk];
   __shared__ int ord_s[kChunk];
@@ -215,26 +393,36 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     __syncthreads();
   }
   if (tid < K) counts[(bh * nchunk + c) * K + tid] = start_s[tid + 1] - start_s[tid];
-  // column sums over the sorted runs of this thread's clusters
-  const int g = tid / D, dcol = tid % D;
-  double* out = partial + (bh * nchunk + c) * K * D + dcol;
+  // column sums over the sorted runs of this group's clusters
+  const int g = tid / LPG, col = 8 * (tid % LPG);
+  double* out = partial + (bh * nchunk + c) * K * D + col;
   const int64_t xrow0 = (b * S + t0) * H + h;
   for (int j = g; j < K; j += NG) {
     const int p1 = start_s[j + 1];
-    double acc = 0.0;
-    constexpr int kPf = 8;
+    double acc[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[k] = 0.0;
+    constexpr int kPf = DT == kF32 ? 4 : 8;
     for (int p0 = start_s[j]; p0 < p1; p0 += kPf) {
-      float v[kPf];
+      Raw8<DT> raw[kPf];
 #pragma unroll
       for (int i = 0; i < kPf; ++i) {
         const int pos = p0 + i < p1 ? p0 + i : p1 - 1;
-        v[i] = load_as_f32(x, (xrow0 + static_cast<int64_t>(ord_s[pos]) * H) * D + dcol, DT);
+        raw[i].load(x, (xrow0 + static_cast<int64_t>(ord_s[pos]) * H) * D + col);
       }
 #pragma unroll
-      for (int i = 0; i < kPf; ++i)
-        if (p0 + i < p1) acc += static_cast<double>(v[i]);
+      for (int i = 0; i < kPf; ++i) {
+        if (p0 + i < p1) {
+          float v[8];
+          raw[i].to_f32(v);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(v[k]);
+        }
+      }
     }
-    out[j * D] = acc;
+    double2* o = reinterpret_cast<double2*>(out + j * D);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
   }
 }
 
@@ -249,9 +437,22 @@ __global__ void km_finalize_kernel(const double* partial, const int32_t* counts,
   if (d >= D || changed[bh] == 0) return;
   double tot = 0.0;
   int64_t cnt = 0;
-  for (int64_t c = 0; c < nchunk; ++c) {
-    tot += partial[((bh * nchunk + c) * K + j) * D + d];
-    cnt += counts[(bh * nchunk + c) * K + j];
+  // 8 chunks' loads in flight, added in chunk order
+  const double* p = partial + (bh * nchunk * K + j) * D + d;
+  const int32_t* pc = counts + bh * nchunk * K + j;
+  for (int64_t c0 = 0; c0 < nchunk; c0 += 8) {
+    double v[8];
+    int32_t n[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int64_t c = c0 + i < nchunk ? c0 + i : nchunk - 1;
+      v[i] = p[c * K * D];
+      n[i] = pc[c * K];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (c0 + i < nchunk) { tot += v[i]; cnt += n[i]; }
+    }
   }
   if (cnt > 0) cent[(bh * K + j) * D + d] = static_cast<float>(tot / static_cast<double>(cnt));
 }
@@ -354,18 +555,25 @@ extern "C" int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64
   hipLaunchKernelGGL(km_init_kernel, dim3(static_cast<unsigned>(BH * K)), dim3(static_cast<unsigned>(D)), 0, st, x,
                      dtype, S, H, D, K, seed, w.cent);
   LBFQ_LAUNCH_CHECK("km_init");
-  const int64_t nblk_s = (S + 255) / 256;
+  // assignment: two workgroups per CU, fewer where there are fewer slabs
+  const int64_t nslabs = BH * ((S + kSlab - 1) / kSlab);
+  const unsigned nasg = static_cast<unsigned>(nslabs < 512 ? nslabs : 512);
   const int rounds = iters > 0 ? iters : 1;
   for (int it = 0; it < rounds; ++it) {
-    const dim3 ga(static_cast<unsigned>(BH * nblk_s)), gu(static_cast<unsigned>(BH * nchunk));
+    const dim3 ga(nasg), gu(static_cast<unsigned>(BH * nchunk));
     // round it writes flag slot it % 2, read by its update and finalize and by
     // round it + 1's assignment; finalize clears slot (it + 1) % 2 first
     int32_t* cur = w.changed + (it & 1) * BH;
     const int32_t* prev = it == 0 ? nullptr : w.changed + ((it - 1) & 1) * BH;
-#define LBFQ_KM(DD, DT)                                                                                     \
-  hipLaunchKernelGGL((km_assign_kernel<DD, DT>), ga, dim3(256), 0, st, x, S, H, K, w.cent, labels, prev, cur); \
-  if (it + 1 < rounds)                                                                                      \
-    hipLaunchKernelGGL((km_update_partial_kernel<DD, DT>), gu, dim3(kUpdThreads), 0, st, x, S, H, K, labels,  \
+#define LBFQ_KM(DD, DT)                                                                                             \
+  if (K <= 32)                                                                                                      \
+    hipLaunchKernelGGL((km_assign_kernel<DD, DT, 1>), ga, dim3(kAsgThreads), 0, st, x, BH, S, H, K, w.cent, labels, \
+                       prev, cur);                                                                                  \
+  else                                                                                                              \
+    hipLaunchKernelGGL((km_assign_kernel<DD, DT, 2>), ga, dim3(kAsgThreads), 0, st, x, BH, S, H, K, w.cent, labels, \
+                       prev, cur);                                                                                  \
+  if (it + 1 < rounds)                                                                                              \
+    hipLaunchKernelGGL((km_update_partial_kernel<DD, DT>), gu, dim3(kUpdThreads), 0, st, x, S, H, K, labels,        \
                        w.partial, w.counts, cur);
     if (D == 128) {
       if (dtype == kBF16) { LBFQ_KM(128, kBF16) } else if (dtype == kF16) { LBFQ_KM(128, kF16) } else { LBFQ_KM(128, kF32) }
