@@ -13,8 +13,14 @@
 // A slice whose assignment leaves every label as it was has converged: its
 // later rounds would recompute the same centroids and labels exactly, so its
 // workgroups skip them (a per-slice flag on the device, no host round trip).
+// Within a slice that still moves, most of a round repeats the previous one:
+// a token whose label cannot have changed (distance bounds, below) is not read
+// again by the assignment, and a chunk whose sums are exact in fp64 is updated
+// by the tokens that moved instead of being summed anew.  Both leave every
+// label and centroid bit as the rounds above define them.
 // The order is a stable counting sort of the labels (argsort stable=True).
 #include <mutex>
+#include <type_traits>
 #include "lbfq_common.h"
 #include "../../include/lbfq.h"
 
@@ -35,8 +41,19 @@ __device__ __forceinline__ uint64_t kmix(uint64_t seed, uint64_t bh, uint64_t K,
   return z ^ (z >> 31);
 }
 
+// State carried from round to round (all null where the workspace has no room for it).
+struct Track {
+  float2* ul;           // [BH][S]: distance bounds of each token when it was last assigned (assign_settle)
+  float* cum;           // [BH][K]: path length of each centroid so far
+  float* delta;         // [BH][K]: its last step
+  float* cum_max;       // [2][BH]: sum over the rounds of the longest step, slot it % 2 read by round it
+  int32_t* touched;     // [BH][K]: an update changed the cluster's sums since the last centroid pass
+  int32_t* exact;       // [BH][nchunk]: every fp64 sum over the chunk's values is exact
+  uint8_t* part_label;  // [BH][S]: the labels that the chunk's partial sums stand for
+};
+
 __global__ void km_init_kernel(const void* x, int dt, int64_t S, int64_t H, int64_t D, int K, uint64_t seed,
-                               float* cent) {
+                               float* cent, float* cum) {
   const int64_t bh = blockIdx.x / K;
   const int j = blockIdx.x % K;
   const int64_t b = bh / H, h = bh % H;
@@ -44,10 +61,12 @@ __global__ void km_init_kernel(const void* x, int dt, int64_t S, int64_t H, int6
   const int64_t idx = j * stride + static_cast<int64_t>(kmix(seed, bh, K, j) % static_cast<uint64_t>(stride));
   const int d = threadIdx.x;
   if (d < D) cent[(bh * K + j) * D + d] = load_as_f32(x, ((b * S + idx) * H + h) * D + d, dt);
+  if (cum && d == 0) cum[bh * K + j] = 0.0f;
 }
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // 8 consecutive elements of dtype DT: as loaded, and as fp32
 template <int DT>
@@ -123,7 +142,8 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& 
 // 278 us with 64 clusters: the FMA issue bound it).
 constexpr int kAsgWaves = 8;
 constexpr int kAsgThreads = 64 * kAsgWaves;
-constexpr int kSlab = 32 * kAsgWaves;  // tokens per step of a workgroup
+constexpr int kSlab = 32 * kAsgWaves;  // tokens per slab: one 32-token step of each wave
+constexpr int kSeg = 4;                // slabs listed at a time
 
 template <int D, int MB>
 struct AssignLds {
@@ -204,148 +224,262 @@ __device__ __forceinline__ int assign_exact(const AssignLds<D, MB>& lds, const v
   return best;
 }
 
+// ---- distance bounds (Hamerly, "Making k-means even faster", SDM 2010) -------------
+// With every assignment a token keeps u >= |x - c_label| and
+// l <= min over the other centroids of |x - c_j|.  A later round's centroids
+// lie at most their path length away, so with cum[j] the length of centroid
+// j's path and cmax the sum over the rounds of the longest step,
+//   |x - c_label| <= u + (cum[label] - cum[label] then),
+//   |x - c_j|     >= l - (cmax - cmax then);
+// u - cum and l + cmax are what is stored.  While the squared distances stay
+// further apart than twice the error of the specification's fp32 scores
+// (2^-16 X C + 2^-17 C^2 each, X <= u + C), the label is what the
+// specification would choose again, and the token's row is not read.  All
+// roundings are taken outwards by 2^-18 relative, 50 times their size.
+constexpr float kOut = 0x1p-18f;
+
+// label still certain: (st.x, st.y) the stored pair, cum and cmax of now, c >= max_j |c_j|
+__device__ __forceinline__ bool bounds_hold(float2 st, float cum, float cmax, float c) {
+  const float u = st.x + cum + kOut * (fabsf(st.x) + cum);
+  const float l = st.y - cmax - kOut * (fabsf(st.y) + cmax);
+  const float thr = 0x1p-14f * (u + c) * c + 0x1p-15f * c * c + 0x1p-120f;
+  return l > u && (l - u) * (l + u) > thr;  // false for NaN
+}
+
 // Grid: any number of workgroups; each takes a contiguous share of the
 // BH * ceil(S / kSlab) slabs (two workgroups per CU and equal shares: no
-// partial last wave of workgroups), refilling LDS when the slice changes.
+// partial last wave of workgroups), up to kSeg slabs of one slice at a time,
+// refilling LDS when the slice changes.  From the second round on it first
+// lists the segment's tokens whose bounds no longer hold, and its waves take
+// 32 of the list at a time.
 // prev_changed: the flags of the previous round (NULL in the first round);
 // changed: this round's flags, set to 1 for a slice in which some label
 // changed.  They are zero on entry from the second round on; in the first
 // round every label counts as changed, so every slice's flag is written.
+// it: the round.
 template <int D, int DT, int MB>
 __global__ void __launch_bounds__(kAsgThreads, 4)
     km_assign_kernel(const void* x, int64_t BH, int64_t S, int64_t H, int K, const float* cent, int32_t* labels,
-                     const int32_t* prev_changed, int32_t* changed) {
+                     const int32_t* prev_changed, int32_t* changed, const Track tr, int it) {
   constexpr int NKS = D / 16;
   constexpr bool XSPLIT = DT != kBF16;
   constexpr float kGapXC = XSPLIT ? 0x1p-13f : 0x1p-14f, kGapCC = XSPLIT ? 0x1p-14f : 0x1p-15f;
   __shared__ AssignLds<D, MB> lds;
+  __shared__ float cum_s[32 * MB];
+  __shared__ int list_s[kSeg * kSlab];
+  __shared__ int nlist_s;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 31, g = lane >> 5;
+  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   const int64_t nslab = (S + kSlab - 1) / kSlab, total = BH * nslab;
   const int64_t w0 = total * blockIdx.x / gridDim.x, w1 = total * (blockIdx.x + 1) / gridDim.x;
+  const bool filter = tr.ul && prev_changed;
   int64_t cur = -1;
-  float c2max = 0.0f;  // >= max_j |c_j|^2
-  for (int64_t w = w0; w < w1; ++w) {
-    const int64_t bh = w / nslab;
+  float c2max = 0.0f, cmax = 0.0f;  // >= max_j |c_j|^2; the slice's cum_max of this round
+  for (int64_t w = w0; w < w1;) {
+    const int64_t bh = w / nslab, s_in = w - bh * nslab;
+    int64_t ns = w1 - w < kSeg ? w1 - w : kSeg;
+    ns = nslab - s_in < ns ? nslab - s_in : ns;
+    w += ns;
     if (prev_changed && prev_changed[bh] == 0) continue;  // converged slice (uniform per workgroup)
     if (bh != cur) {
       if (cur >= 0) __syncthreads();  // every wave is done with the previous slice's centroids
       assign_fill<D, MB>(lds, cent + bh * K * D, K);
       cur = bh;
       c2max = 0.0f;
-      for (int j = 0; j < K; ++j) c2max = fmaxf(c2max, lds.cn[j]);
-      for (int j = 0; j < K; ++j) c2max = lds.cn[j] < INFINITY ? c2max : INFINITY;
+      for (int j = 0; j < K; ++j) c2max = lds.cn[j] < INFINITY ? fmaxf(c2max, lds.cn[j]) : INFINITY;
+      if (tr.ul) {
+        if (static_cast<int>(threadIdx.x) < K) cum_s[threadIdx.x] = tr.cum[bh * K + threadIdx.x];
+        cmax = 0.0f;
+        if (prev_changed) {
+          float step = 0.0f;
+          for (int j = 0; j < K; ++j) {
+            const float dj = tr.delta[bh * K + j];
+            step = dj < INFINITY ? fmaxf(step, dj) : INFINITY;
+          }
+          cmax = tr.cum_max[(it & 1) * BH + bh] + step;
+        }
+        if (s_in == 0 && threadIdx.x == 0) tr.cum_max[((it + 1) & 1) * BH + bh] = cmax;
+        __syncthreads();
+      }
     }
-    const int64_t t0 = (w - bh * nslab) * kSlab + wave * 32;
-    if (t0 >= S) continue;  // no barrier below
+    const int64_t base = s_in * kSlab;  // the segment's first token
+    const int n = static_cast<int>(S - base < ns * kSlab ? S - base : ns * kSlab);
+    int32_t* const lab = labels + bh * S + base;
+    int nl = n;  // tokens to assign
+    if (filter) {
+      __syncthreads();  // every wave is done with the previous list
+      if (threadIdx.x == 0) nlist_s = 0;
+      __syncthreads();
+      const float c = 1.001f * sqrtf(c2max);
+      for (int i0 = 0; i0 < n; i0 += kAsgThreads) {
+        const int i = i0 + static_cast<int>(threadIdx.x);
+        const bool need = i < n && !bounds_hold(tr.ul[bh * S + base + i], cum_s[lab[i]], cmax, c);
+        const uint64_t m = __ballot(need);
+        int at = 0;
+        if (lane == 0 && m) at = atomicAdd(&nlist_s, __popcll(m));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (need) list_s[at + __popcll(m & lt_mask)] = i;
+      }
+      __syncthreads();
+      nl = nlist_s;
+    }
     const int64_t b = bh / H, h = bh - b * H;
-    const int64_t t = t0 + li < S ? t0 + li : S - 1;  // lanes past the end repeat the last token
-    const int64_t x0 = ((b * S + t) * H + h) * D;
-    float xx = 0.0f;
-    v16f a[MB];
+    const int64_t xseg = ((b * S + base) * H + h) * D;
+    for (int p0 = wave * 32; p0 < nl; p0 += 32 * kAsgWaves) {
+      // the centroid operands are read from LDS in every step: kept in registers
+      // across steps they do not fit
+      asm volatile("" ::: "memory");
+      const bool valid = p0 + li < nl;
+      const int p = valid ? p0 + li : nl - 1;  // lanes past the end repeat the last token
+      const int i = filter ? list_s[p] : p;
+      const int64_t x0 = xseg + static_cast<int64_t>(i) * H * D;
+      float xx = 0.0f;
+      v16f a[MB];
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+      for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) a[m][r] = -0.5f * lds.cn[32 * m + 8 * (r >> 2) + 4 * g + (r & 3)];
-    // token operands: lane (li, g) holds dimensions 16 ks + 8 g + [0, 8) of its
-    // token, GK k-steps' loads in flight (all; half with fp32 tokens and 64
-    // centroids, to stay under 128 registers)
-    constexpr int GK = DT == kF32 && MB == 2 && NKS == 8 ? 4 : NKS;
+        for (int r = 0; r < 16; ++r) a[m][r] = -0.5f * lds.cn[32 * m + 8 * (r >> 2) + 4 * g + (r & 3)];
+      // token operands: lane (li, g) holds dimensions 16 ks + 8 g + [0, 8) of its
+      // token, GK k-steps' loads in flight (all; two with fp32 tokens and 64
+      // centroids, to stay under 128 registers)
+      constexpr int GK = DT == kF32 && MB == 2 ? 2 : NKS;
 #pragma unroll 1
-    for (int k0 = 0; k0 < NKS; k0 += GK) {
-      Raw8<DT> raw[GK];
+      for (int k0 = 0; k0 < NKS; k0 += GK) {
+        Raw8<DT> raw[GK];
 #pragma unroll
-      for (int i = 0; i < GK; ++i) raw[i].load(x, x0 + 16 * (k0 + i) + 8 * g);
+        for (int q = 0; q < GK; ++q) raw[q].load(x, x0 + 16 * (k0 + q) + 8 * g);
 #pragma unroll
-      for (int i = 0; i < GK; ++i) {
-        const int ks = k0 + i;
-        float v[8];
-        raw[i].to_f32(v);
-        bf16x8 xh, xl;
-        split8(v, xh, xl);  // of bf16 tokens xl is zero, and unused
+        for (int q = 0; q < GK; ++q) {
+          const int ks = k0 + q;
+          bf16x8 xh, xl;
+          if constexpr (XSPLIT) {
+            float v[8];
+            raw[q].to_f32(v);
+            split8(v, xh, xl);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xx = fmaf(v[e], v[e], xx);
+            for (int e = 0; e < 8; ++e) xx = fmaf(v[e], v[e], xx);
+          } else {
+            xh = __builtin_bit_cast(bf16x8, raw[q].r[0]);
 #pragma unroll
-        for (int m = 0; m < MB; ++m) {
-          const bf16x8 ch = __builtin_bit_cast(bf16x8, lds.part[0][ks][m][lane]);
-          const bf16x8 cl = __builtin_bit_cast(bf16x8, lds.part[1][ks][m][lane]);
-          a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xh, a[m], 0, 0, 0);
-          a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, xh, a[m], 0, 0, 0);
-          if constexpr (XSPLIT) a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xl, a[m], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+              const bf16x2 pr = {xh[2 * e], xh[2 * e + 1]};
+              xx = __builtin_amdgcn_fdot2_f32_bf16(pr, pr, xx, false);
+            }
+          }
+#pragma unroll
+          for (int m = 0; m < MB; ++m) {
+            const bf16x8 ch = __builtin_bit_cast(bf16x8, lds.part[0][ks][m][lane]);
+            const bf16x8 cl = __builtin_bit_cast(bf16x8, lds.part[1][ks][m][lane]);
+            a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xh, a[m], 0, 0, 0);
+            a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, xh, a[m], 0, 0, 0);
+            if constexpr (XSPLIT) a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xl, a[m], 0, 0, 0);
+          }
         }
       }
-    }
-    xx += __shfl_xor(xx, 32, 64);
-    // X C and C^2 from above: 2^-110 covers squares lost to underflow, 1.001 the roundings of the norms
-    const float xc = sqrtf((xx + 0x1p-110f) * (c2max + 0x1p-110f));
-    const float gap = 1.001f * (kGapXC * xc + kGapCC * c2max) + 0x1p-120f;
-    float top = -INFINITY;
+      xx += __shfl_xor(xx, 32, 64);
+      // X C and C^2 from above: 2^-110 covers squares lost to underflow, 1.001 the roundings of the norms
+      const float xc = sqrtf((xx + 0x1p-110f) * (c2max + 0x1p-110f));
+      const float gap = 1.001f * (kGapXC * xc + kGapCC * c2max) + 0x1p-120f;
+      float top = -INFINITY;
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+      for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) top = fmaxf(top, a[m][r]);
-    top = fmaxf(top, __shfl_xor(top, 32, 64));
-    const float thr = top - gap;
-    int cnt = 0, bj = 0;
+        for (int r = 0; r < 16; ++r) top = fmaxf(top, a[m][r]);
+      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      const float thr = top - gap;
+      int cnt = 0, bj = 0;
+      float second = -INFINITY;  // the largest a_j of the others, where one centroid is near
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+      for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const bool near = !(a[m][r] < thr);  // NaN on either side counts as near
-        cnt += near ? 1 : 0;
-        bj = near ? 32 * m + 8 * (r >> 2) + (r & 3) : bj;
-      }
-    bj = cnt ? bj + 4 * g : 0;
-    const int cnt2 = cnt + __shfl_xor(cnt, 32, 64);
-    bj = max(bj, __shfl_xor(bj, 32, 64));  // the one near centroid, if there is one
-    // unsettled tokens, two at a time with up to 32 centroids
-    uint32_t open = static_cast<uint32_t>(__ballot(cnt2 != 1 && t0 + li < S));
-    while (open) {
-      const int i0 = __builtin_ctz(open);
-      open &= open - 1;
-      int i1 = i0;
-      if (MB == 1 && open) {
-        i1 = __builtin_ctz(open);
+        for (int r = 0; r < 16; ++r) {
+          const bool near = !(a[m][r] < thr);  // NaN on either side counts as near
+          cnt += near ? 1 : 0;
+          bj = near ? 32 * m + 8 * (r >> 2) + (r & 3) : bj;
+          second = near ? second : fmaxf(second, a[m][r]);
+        }
+      bj = cnt ? bj + 4 * g : 0;
+      const int cnt2 = cnt + __shfl_xor(cnt, 32, 64);
+      bj = max(bj, __shfl_xor(bj, 32, 64));  // the one near centroid, if there is one
+      second = fmaxf(second, __shfl_xor(second, 32, 64));
+      // unsettled tokens, two at a time with up to 32 centroids
+      const bool unsettled = cnt2 != 1;
+      uint32_t open = static_cast<uint32_t>(__ballot(unsettled && valid));
+      while (open) {
+        const int i0 = __builtin_ctz(open);
         open &= open - 1;
+        int i1 = i0;
+        if (MB == 1 && open) {
+          i1 = __builtin_ctz(open);
+          open &= open - 1;
+        }
+        const int ti = __shfl(i, MB == 1 && lane >= 32 ? i1 : i0, 64);
+        const int le = assign_exact<D, DT, MB>(lds, x, xseg + static_cast<int64_t>(ti) * H * D, lane);
+        const int l0 = __builtin_amdgcn_readlane(le, 0), l1 = __builtin_amdgcn_readlane(le, 32);
+        if (li == i0) bj = l0;
+        else if (li == i1) bj = l1;
       }
-      const int ti = MB == 1 && lane >= 32 ? i1 : i0;
-      const int lab = assign_exact<D, DT, MB>(lds, x, ((b * S + t0 + ti) * H + h) * D, lane);
-      const int l0 = __builtin_amdgcn_readlane(lab, 0), l1 = __builtin_amdgcn_readlane(lab, 32);
-      if (li == i0) bj = l0;
-      else if (li == i1) bj = l1;
-    }
-    if (lane < 32 && t0 + li < S) {
-      int32_t* lp = labels + bh * S + t0 + li;
-      const int32_t old = prev_changed ? *lp : -1;
-      *lp = bj;
-      if (__any(old != bj) && lane == 0) changed[bh] = 1;
+      if (lane < 32 && valid) {
+        const int32_t old = prev_changed ? lab[i] : -1;
+        lab[i] = bj;
+        if (__any(old != bj) && lane == 0) changed[bh] = 1;
+        if (tr.ul) {
+          // |x - c_j|^2 = |x|^2 - 2 a_j, with twice the error of a_j (and that of
+          // the stored norms) below the gap and that of |x|^2 below 2^-15 of it
+          const float e = gap + 0x1p-15f * xx;
+          float2 st = make_float2(INFINITY, 0.0f);  // never holds
+          if (!unsettled) {
+            st.x = sqrtf(fmaxf(xx - 2.0f * top, 0.0f) + e) * (1.0f + kOut) - cum_s[bj];
+            st.y = sqrtf(fmaxf(xx - 2.0f * second - e, 0.0f)) * (1.0f - kOut) + cmax;
+          }
+          tr.ul[bh * S + base + i] = st;
+        }
+      }
     }
   }
 }
 
+// ---- update -------------------------------------------------------------------------
 // fp64 per-cluster column sums of one kChunk-token chunk.  The chunk's tokens
 // are first sorted by label in LDS, stably (ballot ranks within a wave, waves
 // and rounds in token order), so a cluster's tokens keep their order.  Then
 // the D / 8 lanes of group g -- 8 columns each, one 16-byte load per bf16 row --
 // add the runs of clusters j = g, g + NG, ... in that order: the token-order
 // fp64 sums of the specification, with 8 rows in flight per lane.
+//
+// The first round also finds out whether the chunk's sums are exact: values
+// are multiples of the smallest nonzero one's last bit, and a sum of up to
+// 2^12 of them stays below 2^12 times the bound of the largest, so if that
+// span fits fp64's 53 bits no addition rounds and the order does not matter
+// (bf16 normal data spans ~25 of the 33 exponents this leaves).  In an exact
+// chunk a later round adds and subtracts only the tokens whose label differs
+// from the one the partial sums stand for -- the same bits as summing anew --
+// unless more than a quarter of the chunk moved.
+//
 // Bound by the row reads (and the LDS sort ahead of them); with one column and
-// a 2-byte load per lane it took 132 us a round at 40 x 32768 x 128 bf16, 32
-// clusters (2.5 TB/s).
+// a 2-byte load per lane the full sums took 132 us a round at
+// 40 x 32768 x 128 bf16, 32 clusters (2.5 TB/s).
 constexpr int kUpdThreads = 512;
+constexpr int kMaxMoved = kChunk / 4;
 
 template <int D, int DT>
 __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const void* x, int64_t S, int64_t H, int K,
                                                                         const int32_t* labels, double* partial,
-                                                                        int32_t* counts, const int32_t* changed) {
-  constexpr int LPG = D / 8;              // lanes per cluster group
+                                                                        int32_t* counts, const int32_t* changed,
+                                                                        const Track tr, int first) {
+  constexpr int LPG = D / 8;             // lanes per cluster group
   constexpr int NG = kUpdThreads / LPG;  // cluster groups
   constexpr int NW = kUpdThreads / 64;
-  __shared__ int lab_s[kChunk];
-  __shared__ int ord_s[kChunk];
+  constexpr int kPf = DT == kF32 ? 4 : 8;  // rows in flight per lane
+  constexpr int kGone = 1 << 16;           // move entry: the row left the cluster
+  __shared__ int lab_s[kChunk];  // label; moved tokens: + (previous label + 1) << 8
+  __shared__ int ord_s[kChunk];  // rows in cluster order, or the moves in cluster order
   __shared__ int start_s[kMaxKAssign + 1];
   __shared__ int running[kMaxKAssign];
+  __shared__ int net_s[kMaxKAssign];
   __shared__ int wcnt[NW][kMaxKAssign];
+  __shared__ uint32_t range_s[2];  // largest magnitude; smallest nonzero one, minus 1 (fp32 bits)
   const int64_t nchunk = (S + kChunk - 1) / kChunk;
   const int64_t bh = blockIdx.x / nchunk, c = blockIdx.x % nchunk;
   if (changed[bh] == 0) return;  // converged slice (uniform per workgroup)
@@ -353,24 +487,115 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t t0 = c * kChunk;
   const int n = static_cast<int>(t0 + kChunk < S ? kChunk : S - t0);
-  for (int i = tid; i < K; i += kUpdThreads) { start_s[i + 1] = 0; running[i] = 0; }
+  const int g = tid / LPG, col = 8 * (tid % LPG);
+  double* const out = partial + (bh * nchunk + c) * K * D + col;
+  int32_t* const cnt_out = counts + (bh * nchunk + c) * K;
+  const int64_t xrow0 = (b * S + t0) * H + h;
+  const bool by_moves = tr.ul && !first && tr.exact[bh * nchunk + c] != 0;  // if few enough moved
+  for (int i = tid; i < K; i += kUpdThreads) { start_s[i + 1] = 0; running[i] = 0; net_s[i] = 0; }
   for (int i = tid; i < NW * K; i += kUpdThreads) wcnt[i / K][i % K] = 0;
-  for (int i = tid; i < n; i += kUpdThreads) lab_s[i] = labels[bh * S + t0 + i];
+  if (tid < 2) range_s[tid] = tid ? 0xffffffffu : 0u;
+  int moved = 0;
+  for (int r0 = 0; r0 < kChunk; r0 += kUpdThreads) {
+    const int i = r0 + tid;
+    bool mv = false;
+    if (i < n) {
+      const int L = labels[bh * S + t0 + i];
+      int old = 0;
+      if (tr.ul) {
+        uint8_t* pl = tr.part_label + bh * S + t0 + i;
+        if (by_moves) {
+          old = *pl;
+          mv = old != L;
+        }
+        if (!by_moves || mv) *pl = static_cast<uint8_t>(L);
+      }
+      lab_s[i] = mv ? L | (old + 1) << 8 : L;
+    }
+    if (by_moves) moved += __syncthreads_count(mv);
+  }
+  if (by_moves && moved == 0) return;
+  const bool moves = by_moves && moved <= kMaxMoved;
   __syncthreads();
-  for (int i = tid; i < n; i += kUpdThreads) atomicAdd(&start_s[lab_s[i] + 1], 1);
-  __syncthreads();
-  if (tid == 0) {
-    start_s[0] = 0;
-    for (int j = 0; j < K; ++j) start_s[j + 1] += start_s[j];
+  // histogram and starts of the clusters' runs
+  for (int i = tid; i < n; i += kUpdThreads) {
+    const int v = lab_s[i], L = v & 0xff, old = (v >> 8) - 1;
+    if (!moves) {
+      atomicAdd(&start_s[L + 1], 1);
+    } else if (old >= 0) {
+      atomicAdd(&start_s[L + 1], 1);
+      atomicAdd(&start_s[old + 1], 1);
+      atomicAdd(&net_s[L], 1);
+      atomicAdd(&net_s[old], -1);
+    }
   }
   __syncthreads();
+  if (wave == 0) {  // inclusive scan; K <= 64
+    int v = lane < K ? start_s[lane + 1] : 0;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      const int o = __shfl_up(v, m, 64);
+      v += lane >= m ? o : 0;
+    }
+    if (lane < K) start_s[lane + 1] = v;
+    if (lane == 0) start_s[0] = 0;
+  }
+  __syncthreads();
+  if (moves) {  // entries of a cluster in any order: their sums are exact
+    for (int i = tid; i < n; i += kUpdThreads) {
+      const int v = lab_s[i], L = v & 0xff, old = (v >> 8) - 1;
+      if (old >= 0) {
+        ord_s[start_s[L] + atomicAdd(&running[L], 1)] = i;
+        ord_s[start_s[old] + atomicAdd(&running[old], 1)] = i | kGone;
+      }
+    }
+    __syncthreads();
+    if (tid < K && start_s[tid + 1] > start_s[tid]) {
+      cnt_out[tid] += net_s[tid];
+      tr.touched[bh * K + tid] = 1;
+    }
+    for (int j = g; j < K; j += NG) {
+      const int p1 = start_s[j + 1];
+      int p0 = start_s[j];
+      if (p0 == p1) continue;
+      double2* o = reinterpret_cast<double2*>(out + j * D);
+      double acc[8];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const double2 v = o[k];
+        acc[2 * k] = v.x;
+        acc[2 * k + 1] = v.y;
+      }
+      for (; p0 < p1; p0 += kPf) {
+        Raw8<DT> raw[kPf];
+#pragma unroll
+        for (int i = 0; i < kPf; ++i) {
+          const int r = ord_s[p0 + i < p1 ? p0 + i : p1 - 1] & (kGone - 1);
+          raw[i].load(x, (xrow0 + static_cast<int64_t>(r) * H) * D + col);
+        }
+#pragma unroll
+        for (int i = 0; i < kPf; ++i) {
+          if (p0 + i < p1) {
+            float v[8];
+            raw[i].to_f32(v);
+            const float sg = ord_s[p0 + i] & kGone ? -1.0f : 1.0f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(sg * v[k]);
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
+    }
+    return;
+  }
   int nbits = 1;
   while ((1 << nbits) < K) ++nbits;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   for (int r0 = 0; r0 < n; r0 += kUpdThreads) {
     const int r = r0 + tid;
     const bool valid = r < n;
-    const int L = valid ? lab_s[r] : -1;
+    const int L = valid ? lab_s[r] & 0xff : -1;
     uint64_t match = __ballot(valid);
     for (int bit = 0; bit < nbits; ++bit) {
       const uint64_t bal = __ballot(valid && ((L >> bit) & 1));
@@ -392,17 +617,17 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     }
     __syncthreads();
   }
-  if (tid < K) counts[(bh * nchunk + c) * K + tid] = start_s[tid + 1] - start_s[tid];
+  if (tid < K) {
+    cnt_out[tid] = start_s[tid + 1] - start_s[tid];
+    if (tr.ul) tr.touched[bh * K + tid] = 1;
+  }
   // column sums over the sorted runs of this group's clusters
-  const int g = tid / LPG, col = 8 * (tid % LPG);
-  double* out = partial + (bh * nchunk + c) * K * D + col;
-  const int64_t xrow0 = (b * S + t0) * H + h;
+  uint32_t big = 0u, small = 0xffffffffu;
   for (int j = g; j < K; j += NG) {
     const int p1 = start_s[j + 1];
     double acc[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) acc[k] = 0.0;
-    constexpr int kPf = DT == kF32 ? 4 : 8;
     for (int p0 = start_s[j]; p0 < p1; p0 += kPf) {
       Raw8<DT> raw[kPf];
 #pragma unroll
@@ -417,6 +642,14 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
           raw[i].to_f32(v);
 #pragma unroll
           for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(v[k]);
+          if (first) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const uint32_t a = __float_as_uint(v[k]) & 0x7fffffffu;
+              big = a > big ? a : big;
+              small = a - 1u < small ? a - 1u : small;  // 0 - 1 wraps to the top
+            }
+          }
         }
       }
     }
@@ -424,20 +657,42 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
 #pragma unroll
     for (int k = 0; k < 4; ++k) o[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
   }
+  if (tr.ul && first) {
+    atomicMax(&range_s[0], big);
+    atomicMin(&range_s[1], small);
+    __syncthreads();
+    if (tid == 0) {
+      // mantissa bits below the leading one of a value of this dtype
+      constexpr int kMant = DT == kF32 ? 23 : DT == kF16 ? 10 : 7;
+      const int eb = static_cast<int>(range_s[0] >> 23);  // biased exponents
+      int es = static_cast<int>((range_s[1] + 1u) >> 23);
+      es = es < 1 ? 1 : es;
+      // 2^(eb + 1) * 2^12 terms over a last bit of 2^(es - kMant): 53 bits hold them
+      tr.exact[bh * nchunk + c] = eb < 255 && (range_s[0] == 0u || eb + 1 + 12 - (es - kMant) <= 53) ? 1 : 0;
+    }
+  }
 }
 
 // changed: this round's flags; clear_next: the next round's, cleared here
-// (the previous round's assignment, their last reader, has finished).
-__global__ void km_finalize_kernel(const double* partial, const int32_t* counts, int64_t nchunk, int K, int64_t D,
-                                   float* cent, const int32_t* changed, int32_t* clear_next) {
+// (the previous round's assignment, their last reader, has finished).  One
+// workgroup per cluster: the chunk sums in chunk order, 8 chunks' loads in
+// flight; a cluster that no chunk touched keeps its centroid.
+template <int D>
+__global__ void __launch_bounds__(D) km_finalize_kernel(const double* partial, const int32_t* counts, int64_t nchunk,
+                                                        int K, float* cent, const int32_t* changed,
+                                                        int32_t* clear_next, const Track tr) {
+  __shared__ float red[2];
   const int64_t bh = blockIdx.x / K;
   const int j = blockIdx.x % K;
   const int d = threadIdx.x;
   if (j == 0 && d == 0) clear_next[bh] = 0;
-  if (d >= D || changed[bh] == 0) return;
+  if (changed[bh] == 0) return;
+  if (tr.ul && tr.touched[bh * K + j] == 0) {
+    if (d == 0) tr.delta[bh * K + j] = 0.0f;
+    return;
+  }
   double tot = 0.0;
   int64_t cnt = 0;
-  // 8 chunks' loads in flight, added in chunk order
   const double* p = partial + (bh * nchunk * K + j) * D + d;
   const int32_t* pc = counts + bh * nchunk * K + j;
   for (int64_t c0 = 0; c0 < nchunk; c0 += 8) {
@@ -454,7 +709,24 @@ __global__ void km_finalize_kernel(const double* partial, const int32_t* counts,
       if (c0 + i < nchunk) { tot += v[i]; cnt += n[i]; }
     }
   }
-  if (cnt > 0) cent[(bh * K + j) * D + d] = static_cast<float>(tot / static_cast<double>(cnt));
+  float* cp = cent + (bh * K + j) * D + d;
+  const float old = *cp;
+  const float now = cnt > 0 ? static_cast<float>(tot / static_cast<double>(cnt)) : old;
+  *cp = now;
+  if (tr.ul) {  // the length of the centroid's step, from above
+    float s = (now - old) * (now - old);
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m, 64);
+    if ((d & 63) == 0) red[d >> 6] = s;
+    __syncthreads();  // also: every thread has read touched
+    if (d == 0) {
+      if (D == 128) s += red[1];
+      const float step = 1.001f * sqrtf(s + 0x1p-120f);
+      tr.delta[bh * K + j] = step;
+      tr.cum[bh * K + j] += step;
+      tr.touched[bh * K + j] = 0;
+    }
+  }
 }
 
 // Stable counting sort of one slice's labels: order[pos] = t, inverse[t] = pos.
@@ -514,51 +786,73 @@ struct KmWs {
   double* partial;
   int32_t* counts;
   int32_t* changed;  // [2][BH]: the convergence flags of two consecutive rounds
+  Track track;
 };
 
-KmWs carve(void* ws, int64_t BH, int64_t S, int64_t D, int K) {
+// The workspace's pieces in order and its size; with `tracked` the state of
+// struct Track follows the rest (its pointers stay null otherwise).
+int64_t carve(void* ws, int64_t BH, int64_t S, int64_t D, int K, bool tracked, KmWs* w) {
   const int64_t nchunk = (S + kChunk - 1) / kChunk;
-  uint8_t* p = static_cast<uint8_t*>(ws);
-  KmWs w;
-  w.partial = reinterpret_cast<double*>(p);
-  p += sizeof(double) * BH * nchunk * K * D;
-  w.cent = reinterpret_cast<float*>(p);
-  p += sizeof(float) * BH * K * D;
-  w.counts = reinterpret_cast<int32_t*>(p);
-  p += sizeof(int32_t) * BH * nchunk * K;
-  w.changed = reinterpret_cast<int32_t*>(p);
-  return w;
+  int64_t at = 0;
+  auto take = [&](auto*& ptr, int64_t count) {
+    if (w) ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(static_cast<uint8_t*>(ws) + at);
+    at += count * static_cast<int64_t>(sizeof(*ptr));
+  };
+  KmWs none{};
+  KmWs& k = w ? *w : none;
+  take(k.partial, BH * nchunk * K * D);
+  take(k.cent, BH * K * D);
+  take(k.counts, BH * nchunk * K);
+  take(k.changed, 2 * BH);
+  if (tracked) {
+    at = (at + 7) / 8 * 8;
+    take(k.track.ul, BH * S);
+    take(k.track.cum, BH * K);
+    take(k.track.delta, BH * K);
+    take(k.track.cum_max, 2 * BH);
+    take(k.track.touched, BH * K);
+    take(k.track.exact, BH * nchunk);
+    take(k.track.part_label, BH * S);
+  }
+  return at;
 }
+
+int kmeans_run(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int K, int iters, uint64_t seed,
+               void* workspace, bool tracked, int32_t* labels, int32_t* order, int32_t* inverse, hipStream_t st);
 
 }  // namespace
 
 extern "C" int64_t lbfq_kmeans_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int K) {
-  const int64_t nchunk = (S + kChunk - 1) / kChunk;
-  const int64_t BH = B * H;
-  return sizeof(double) * BH * nchunk * K * D + sizeof(float) * BH * K * D + sizeof(int32_t) * BH * nchunk * K +
-         sizeof(int32_t) * 2 * BH;
+  return carve(nullptr, B * H, S, D, K, true, nullptr);
 }
 
 extern "C" int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int K, int iters,
                            uint64_t seed, void* workspace, int32_t* labels, int32_t* order, int32_t* inverse,
                            lbfq_stream_t stream) {
+  return kmeans_run(x, dtype, B, S, H, D, K, iters, seed, workspace, true, labels, order, inverse,
+                    static_cast<hipStream_t>(stream));
+}
+
+namespace {
+int kmeans_run(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int K, int iters, uint64_t seed,
+               void* workspace, bool tracked, int32_t* labels, int32_t* order, int32_t* inverse, hipStream_t st) {
   LBFQ_CHECK_ARG(x && workspace && labels && order && inverse, "lbfq_kmeans: null pointer");
   LBFQ_CHECK_ARG(D == 64 || D == 128, "lbfq_kmeans: D must be 64 or 128; got %lld", (long long)D);
   LBFQ_CHECK_ARG(dtype >= 0 && dtype <= 2, "lbfq_kmeans: bad dtype %d", dtype);
   LBFQ_CHECK_ARG(K >= 1 && K <= S, "n_clusters must be in [1, S]; got %d for S=%lld", K, (long long)S);
   LBFQ_CHECK_ARG(K <= kMaxKAssign, "lbfq_kmeans: at most %d clusters are supported; got %d", kMaxKAssign, K);
   LBFQ_CHECK_ARG(B * H < (1ll << 31) / 1024, "lbfq_kmeans: too many slices");
-  hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t BH = B * H;
   const int64_t nchunk = (S + kChunk - 1) / kChunk;
-  KmWs w = carve(workspace, BH, S, D, K);
+  const int rounds = iters > 0 ? iters : 1;
+  KmWs w{};
+  carve(workspace, BH, S, D, K, tracked && rounds > 1, &w);  // one round has nothing to carry over
   hipLaunchKernelGGL(km_init_kernel, dim3(static_cast<unsigned>(BH * K)), dim3(static_cast<unsigned>(D)), 0, st, x,
-                     dtype, S, H, D, K, seed, w.cent);
+                     dtype, S, H, D, K, seed, w.cent, w.track.cum);
   LBFQ_LAUNCH_CHECK("km_init");
   // assignment: two workgroups per CU, fewer where there are fewer slabs
   const int64_t nslabs = BH * ((S + kSlab - 1) / kSlab);
   const unsigned nasg = static_cast<unsigned>(nslabs < 512 ? nslabs : 512);
-  const int rounds = iters > 0 ? iters : 1;
   for (int it = 0; it < rounds; ++it) {
     const dim3 ga(nasg), gu(static_cast<unsigned>(BH * nchunk));
     // round it writes flag slot it % 2, read by its update and finalize and by
@@ -568,13 +862,13 @@ extern "C" int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64
 #define LBFQ_KM(DD, DT)                                                                                             \
   if (K <= 32)                                                                                                      \
     hipLaunchKernelGGL((km_assign_kernel<DD, DT, 1>), ga, dim3(kAsgThreads), 0, st, x, BH, S, H, K, w.cent, labels, \
-                       prev, cur);                                                                                  \
+                       prev, cur, w.track, it);                                                                     \
   else                                                                                                              \
     hipLaunchKernelGGL((km_assign_kernel<DD, DT, 2>), ga, dim3(kAsgThreads), 0, st, x, BH, S, H, K, w.cent, labels, \
-                       prev, cur);                                                                                  \
+                       prev, cur, w.track, it);                                                                     \
   if (it + 1 < rounds)                                                                                              \
     hipLaunchKernelGGL((km_update_partial_kernel<DD, DT>), gu, dim3(kUpdThreads), 0, st, x, S, H, K, labels,        \
-                       w.partial, w.counts, cur);
+                       w.partial, w.counts, cur, w.track, it == 0);
     if (D == 128) {
       if (dtype == kBF16) { LBFQ_KM(128, kBF16) } else if (dtype == kF16) { LBFQ_KM(128, kF16) } else { LBFQ_KM(128, kF32) }
     } else {
@@ -583,8 +877,14 @@ extern "C" int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64
 #undef LBFQ_KM
     LBFQ_LAUNCH_CHECK("km_assign / km_update_partial");
     if (it + 1 == rounds) break;  // the last update does not change the labels
-    hipLaunchKernelGGL(km_finalize_kernel, dim3(static_cast<unsigned>(BH * K)), dim3(static_cast<unsigned>(D)), 0, st,
-                       w.partial, w.counts, nchunk, K, D, w.cent, cur, w.changed + ((it + 1) & 1) * BH);
+    int32_t* clear = w.changed + ((it + 1) & 1) * BH;
+    const dim3 gf(static_cast<unsigned>(BH * K));
+    if (D == 128)
+      hipLaunchKernelGGL(km_finalize_kernel<128>, gf, dim3(128), 0, st, w.partial, w.counts, nchunk, K, w.cent, cur,
+                         clear, w.track);
+    else
+      hipLaunchKernelGGL(km_finalize_kernel<64>, gf, dim3(64), 0, st, w.partial, w.counts, nchunk, K, w.cent, cur,
+                         clear, w.track);
     LBFQ_LAUNCH_CHECK("km_finalize");
   }
   hipLaunchKernelGGL(km_sort_kernel, dim3(static_cast<unsigned>(BH)), dim3(kSortThreads), 0, st, labels, S, K, order,
@@ -592,6 +892,7 @@ extern "C" int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64
   LBFQ_LAUNCH_CHECK("km_sort");
   return 0;
 }
+}  // namespace
 
 // ---- allocation-free variant -------------------------------------------------
 // For callers that cannot allocate device memory (code under HIP graph capture,
@@ -600,7 +901,9 @@ extern "C" int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64
 // Its device address is looked up once per device (hipGetSymbolAddress, with
 // that device current) and kept; host code never uses the array's name as an
 // address.  Calls that overlap on one GPU share the array and race.  The
-// kernels write every workspace word they read, so nothing is cleared.
+// kernels write every workspace word they read, so nothing is cleared.  A
+// problem whose centroids and sums fit the array but not the state carried
+// between rounds as well runs without that state.
 constexpr int64_t kKmScratchBytes = int64_t{64} << 20;  // 64 MiB: the 14B Q k-means (40 x 32768, K=32) needs 43 MB
 static __device__ __align__(256) uint8_t scratch[kKmScratchBytes];
 namespace {
@@ -634,7 +937,7 @@ extern "C" int lbfq_kmeans_noalloc(const void* x, int dtype, int64_t B, int64_t 
                                    int iters, uint64_t seed, int32_t* labels, int32_t* order, int32_t* inverse,
                                    lbfq_stream_t stream) {
   LBFQ_CHECK_ARG(B > 0 && S > 0 && H > 0 && D > 0 && K > 0, "lbfq_kmeans_noalloc: empty shape");
-  const int64_t need = lbfq_kmeans_workspace_bytes(B, S, H, D, K);
+  const int64_t need = carve(nullptr, B * H, S, D, K, false, nullptr);
   LBFQ_CHECK_ARG(need <= kKmScratchBytes,
                  "lbfq_kmeans_noalloc: the problem needs %lld bytes of workspace, above the %lld-byte built-in "
                  "scratch; use lbfq_kmeans with a caller workspace",
@@ -642,5 +945,7 @@ extern "C" int lbfq_kmeans_noalloc(const void* x, int dtype, int64_t B, int64_t 
   void* ws = nullptr;
   const int rc = km_scratch_ptr(&ws);
   if (rc) return rc;
-  return lbfq_kmeans(x, dtype, B, S, H, D, K, iters, seed, ws, labels, order, inverse, stream);
+  const bool tracked = lbfq_kmeans_workspace_bytes(B, S, H, D, K) <= kKmScratchBytes;
+  return kmeans_run(x, dtype, B, S, H, D, K, iters, seed, ws, tracked, labels, order, inverse,
+                    static_cast<hipStream_t>(stream));
 }

@@ -51,3 +51,49 @@ def test_undecided_tokens(gpu, kind, dtype):
     else:
         x[0, 3, 0, 5], x[0, 70, 0, 0], x[0, 400, 1, 127] = float("nan"), float("inf"), -float("inf")
     _check(x.to(dtype), gpu, 40)
+
+
+@pytest.mark.parametrize("kind", ["clustered", "drifting", "outlier_scale", "signed_zeros"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_rounds_that_reuse_the_last(gpu, kind, dtype):
+    """Later rounds read only the tokens whose label may change and update
+    exact chunks by their moved tokens (fp32 and wide-range chunks are summed
+    anew): every round count gives the labels of the full rounds, from few moves
+    a round to most of a chunk, over chunk and slab edges."""
+    g = torch.Generator().manual_seed(21)
+    s, h, d, k = 2309, 2, 128, 32
+    if kind == "drifting":   # one slow blob: centroids keep moving, few tokens are certain
+        x = torch.randn(1, s, h, d, generator=g)
+        x[..., 0] = torch.linspace(-20, 20, s)[None, :, None]
+    else:
+        cent = 3 * torch.randn(h, k, d, generator=g)
+        pick = torch.randint(0, k, (s, h), generator=g)
+        x = (torch.stack([cent[i][pick[:, i]] for i in range(h)], 1) + torch.randn(s, h, d, generator=g))[None]
+    if kind == "outlier_scale":   # chunk 0's values span more than fp64 holds exactly
+        x[0, 100, :, 3], x[0, 200, :, 4] = 2.0 ** 14, 2.0 ** -24
+        x[0, 300, 1, 5] = 1e-30
+    elif kind == "signed_zeros":
+        x = torch.where(torch.rand(x.shape, generator=g) < 0.7, -0.0 * x, x)
+    for iters in (2, 3, 12):
+        _check(x.to(dtype), gpu, k, iters=iters, seed=iters)
+
+
+def test_noalloc_without_room_for_the_carried_state(gpu):
+    """A problem that fits the built-in scratch only without the state carried
+    between rounds still runs there, with the same labels."""
+    from low_bit_fake_quant import _lib as L
+    lib = L.load()
+    b, s, h, d, k = 1, 60 << 16, 2, 64, 8
+    need = int(lib.lbfq_kmeans_workspace_bytes(b, s, h, d, k))
+    assert need > int(lib.lbfq_kmeans_noalloc_max_workspace_bytes())
+    x = torch.randn(b, s, h, d, device=gpu, dtype=torch.bfloat16)
+    st = L.stream_handle(gpu)
+    outs = [[torch.full((b * h, s), -1, dtype=torch.int32, device=gpu) for _ in range(3)] for _ in range(2)]
+    L.check(lib.lbfq_kmeans_noalloc(x.data_ptr(), L.DTYPE_CODE[x.dtype], b, s, h, d, k, 4, 0,
+                                    *(t.data_ptr() for t in outs[0]), st), "lbfq_kmeans_noalloc")
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu)
+    L.check(lib.lbfq_kmeans(x.data_ptr(), L.DTYPE_CODE[x.dtype], b, s, h, d, k, 4, 0, ws.data_ptr(),
+                            *(t.data_ptr() for t in outs[1]), st), "lbfq_kmeans")
+    torch.cuda.synchronize()
+    for got, want in zip(*outs):
+        assert torch.equal(got, want)
