@@ -64,14 +64,42 @@ __global__ void km_init_kernel(const void* x, int dt, int64_t S, int64_t H, int6
   if (cum && d == 0) cum[bh * K + j] = 0.0f;
 }
 
+// the larger of two finite numbers in one instruction (fmaxf of values the
+// compiler cannot trace quiets both first; callers test for NaN themselves)
+__device__ __forceinline__ float vmax(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 3.402823466e38f); }
+
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // 8 consecutive elements of dtype DT: as loaded, and as fp32
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x1 __attribute__((ext_vector_type(1)));
 template <int DT>
 struct Raw8 {
   uint4 r[DT == kF32 ? 2 : 1];
+  // magnitudes of a word's values: bits without the sign, two 16-bit values side by side
+  using Mag = std::conditional_t<DT == kF32, u32x1, u16x2>;
+  static __device__ __forceinline__ void range_word(uint32_t w, Mag& big, Mag& small) {
+    const Mag a = __builtin_bit_cast(Mag, w & (DT == kF32 ? 0x7fffffffu : 0x7fff7fffu));
+    big = __builtin_elementwise_max(big, a);
+    const Mag one = 1;
+    small = __builtin_elementwise_min(small, static_cast<Mag>(a - one));  // 0 - 1 wraps to the top
+  }
+  // fold the 8 values into the largest magnitude and the smallest nonzero one, minus 1
+  __device__ __forceinline__ void range(Mag& big, Mag& small) const {
+#pragma unroll
+    for (int k = 0; k < (DT == kF32 ? 2 : 1); ++k) {
+      range_word(r[k].x, big, small);
+      range_word(r[k].y, big, small);
+      range_word(r[k].z, big, small);
+      range_word(r[k].w, big, small);
+    }
+  }
+  static __device__ __forceinline__ uint32_t widest(Mag m, bool largest) {
+    if constexpr (DT == kF32) return m[0];
+    else return largest ? (m[0] > m[1] ? m[0] : m[1]) : (m[0] < m[1] ? m[0] : m[1]);
+  }
   __device__ __forceinline__ void load(const void* x, int64_t idx) {
     const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(x) + idx * (DT == kF32 ? 4 : 2));
     r[0] = p[0];
@@ -127,23 +155,34 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& 
 //   operands split in two            2^-18 X C       (3 * 2^-18 X C when x is split too: the
 //                                                     residuals of both and the lo * lo term)
 //   accumulation                     2^-20 (X C + C^2 / 2) per MFMA: 16, or 24 with x split
-// the last at twice the largest error of an MFMA measured on a gfx950 relative
-// to the magnitudes it adds (2^-21.4 over operands of mixed magnitude, 2^-23
-// over operands of one).  Twice their sum is below 2^-14 X C + 2^-15 C^2
-// (2^-13 and 2^-14 with x split): two centroids whose a_j are further apart
-// than that gap are in the specification's order.  A token with another
-// centroid within the gap of its best -- or with a non-finite value anywhere,
-// since the test counts the centroids that are NOT below the gap -- is settled
-// by the specification itself: one lane per centroid runs the FMA chain, and
-// the wave takes the first minimum.
+//   the centroid's number            2^-17 (X C + C^2 / 2): it replaces a_j's last six bits,
+//                                    so that the largest a_j names its centroid
+// the accumulation at twice the largest error of an MFMA measured on a gfx950
+// relative to the magnitudes it adds (2^-21.4 over operands of mixed magnitude,
+// 2^-23 over operands of one).  Twice their sum is below 1.25 * 2^-14 X C +
+// 2^-15 C^2 (2^-13 and 2^-14 with x split): two centroids whose a_j are further
+// apart than that gap are in the specification's order.  A token with another
+// centroid within the gap of its best -- or with a gap that is not finite, as
+// any non-finite or overflowing product makes it -- is settled by the
+// specification itself.  Where two centroids are near, the usual case,
+// the token waits for the end of the segment: there a wave runs the FMA chains
+// of 32 waiting tokens, one lane for each of their two centroids (a chain is
+// ~4000 cycles of latency; run where each token turned up, one or two of 32,
+// they doubled the kernel's time).  Any more, and one lane per centroid runs
+// the chains at once.
 //
-// Bound by the token reads: 40 x 32768 x 128 bf16 (335 MB a round) with 32
-// clusters took 196 us as one token per lane against LDS broadcasts (1.7 TB/s;
-// 278 us with 64 clusters: the FMA issue bound it).
+// At 40 x 32768 x 128 bf16 (335 MB, 62 us as reads alone in this pattern) a
+// full round takes 118 us with 32 clusters and 105 with 64; one token per lane
+// against LDS broadcasts, bound by its FMA issue, took 196 and 345.  The rest
+// is ~27 us of latency before the first tokens (centroids, bounds, lists),
+// which is also what a late round with few open tokens takes.  A step issues
+// three VALU instructions per centroid and token pair of lanes (number in,
+// second, first); with separate passes for the maximum, the near mask and the
+// runner-up it issued eight and took 121 us with 64 clusters.
 constexpr int kAsgWaves = 8;
 constexpr int kAsgThreads = 64 * kAsgWaves;
 constexpr int kSlab = 32 * kAsgWaves;  // tokens per slab: one 32-token step of each wave
-constexpr int kSeg = 4;                // slabs listed at a time
+constexpr int kSeg = 8;                // slabs of a segment at most
 
 template <int D, int MB>
 struct AssignLds {
@@ -151,6 +190,7 @@ struct AssignLds {
   uint4 part[2][D / 16][MB][64];   // hi / lo operands, as the lanes read them
   float cent[32 * MB * P];
   float cn[32 * MB];
+  float a0[32 * MB];               // -cn / 2, the MFMA accumulators' start; far below any other for rows >= K
 };
 
 // The centroids of slice bh into LDS: fp32 rows, hi / lo MFMA operands and the
@@ -184,9 +224,29 @@ __device__ __forceinline__ void assign_fill(AssignLds<D, MB>& lds, const float* 
       acc = fmaf(v.z, v.z, acc);
       acc = fmaf(v.w, v.w, acc);
     }
-    lds.cn[threadIdx.x] = static_cast<int>(threadIdx.x) < K ? acc : INFINITY;
+    const bool real = static_cast<int>(threadIdx.x) < K;
+    lds.cn[threadIdx.x] = real ? acc : INFINITY;
+    lds.a0[threadIdx.x] = real ? -0.5f * acc : -1e38f;
   }
   __syncthreads();
+}
+
+// v of lane l ^ 32, on the VALU (v_permlane32_swap exchanges the upper half of
+// its first operand with the lower half of its second)
+__device__ __forceinline__ uint32_t from_pair(uint32_t v, int g) {
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return g ? r[0] : r[1];
+}
+__device__ __forceinline__ float from_pair(float v, int g) {
+  return __uint_as_float(from_pair(__float_as_uint(v), g));
+}
+
+// The largest of the lanes' values, which are not negative; infinity if one is not finite.
+__device__ __forceinline__ float wave_top(float v) {
+  v = v < INFINITY ? v : INFINITY;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
+  return v;
 }
 
 // The specification for one token (its row at element x0) per PER lanes: lane
@@ -198,7 +258,7 @@ __device__ __forceinline__ int assign_exact(const AssignLds<D, MB>& lds, const v
   const int j = lane % PER;
   const float* c = lds.cent + j * AssignLds<D, MB>::P;
   float dot = 0.0f;
-#pragma unroll 4
+#pragma unroll 1
   for (int d = 0; d < D; d += 8) {
     float xv[8];
     load8<DT>(x, x0 + d, xv);
@@ -222,6 +282,35 @@ __device__ __forceinline__ int assign_exact(const AssignLds<D, MB>& lds, const v
     if (so < sc || (so == sc && bo < best)) { sc = so; best = bo; }
   }
   return best;
+}
+
+// The specification between centroids j0 < j1 of a token: lane l runs the chain
+// of j0 and lane l ^ 32 that of j1 (j: this lane's); both return the label.  A
+// NaN score never wins, and if nothing does the label is the lower one (0: only
+// centroids 0 and 1 of 2 can both be near a non-finite token).
+template <int D, int DT, int MB>
+__device__ __forceinline__ int assign_pair(const AssignLds<D, MB>& lds, const void* x, int64_t x0, int j) {
+  const float* c = lds.cent + j * AssignLds<D, MB>::P;
+  float dot = 0.0f;
+#pragma unroll 4
+  for (int d = 0; d < D; d += 8) {
+    float xv[8];
+    load8<DT>(x, x0 + d, xv);
+    const float4 c0 = *reinterpret_cast<const float4*>(c + d), c1 = *reinterpret_cast<const float4*>(c + d + 4);
+    dot = fmaf(xv[0], c0.x, dot);
+    dot = fmaf(xv[1], c0.y, dot);
+    dot = fmaf(xv[2], c0.z, dot);
+    dot = fmaf(xv[3], c0.w, dot);
+    dot = fmaf(xv[4], c1.x, dot);
+    dot = fmaf(xv[5], c1.y, dot);
+    dot = fmaf(xv[6], c1.z, dot);
+    dot = fmaf(xv[7], c1.w, dot);
+  }
+  float sc = fmaf(-2.0f, dot, lds.cn[j]);
+  sc = sc < INFINITY ? sc : INFINITY;
+  const float so = __shfl_xor(sc, 32, 64);
+  const int jo = __shfl_xor(j, 32, 64);
+  return so < sc || (so == sc && jo < j) ? jo : j;
 }
 
 // ---- distance bounds (Hamerly, "Making k-means even faster", SDM 2010) -------------
@@ -263,12 +352,13 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
                      const int32_t* prev_changed, int32_t* changed, const Track tr, int it) {
   constexpr int NKS = D / 16;
   constexpr bool XSPLIT = DT != kBF16;
-  constexpr float kGapXC = XSPLIT ? 0x1p-13f : 0x1p-14f, kGapCC = XSPLIT ? 0x1p-14f : 0x1p-15f;
+  constexpr float kGapXC = XSPLIT ? 0x1p-13f : 1.25f * 0x1p-14f, kGapCC = XSPLIT ? 0x1p-14f : 0x1p-15f;
   __shared__ AssignLds<D, MB> lds;
   __shared__ float cum_s[32 * MB];
-  __shared__ int list_s[kSeg * kSlab];
-  __shared__ int nlist_s;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ uint16_t list_s[kSeg * kSlab];  // the segment's tokens to assign
+  __shared__ uint32_t pend_s[kSeg * kSlab];  // tokens between two centroids: token | j0 << 16 | j1 << 24
+  __shared__ int nlist_s, npend_s;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 31, g = lane >> 5;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   const int64_t nslab = (S + kSlab - 1) / kSlab, total = BH * nslab;
@@ -286,19 +376,12 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
       if (cur >= 0) __syncthreads();  // every wave is done with the previous slice's centroids
       assign_fill<D, MB>(lds, cent + bh * K * D, K);
       cur = bh;
-      c2max = 0.0f;
-      for (int j = 0; j < K; ++j) c2max = lds.cn[j] < INFINITY ? fmaxf(c2max, lds.cn[j]) : INFINITY;
+      c2max = wave_top(lane < K ? lds.cn[lane] : 0.0f);
       if (tr.ul) {
         if (static_cast<int>(threadIdx.x) < K) cum_s[threadIdx.x] = tr.cum[bh * K + threadIdx.x];
         cmax = 0.0f;
-        if (prev_changed) {
-          float step = 0.0f;
-          for (int j = 0; j < K; ++j) {
-            const float dj = tr.delta[bh * K + j];
-            step = dj < INFINITY ? fmaxf(step, dj) : INFINITY;
-          }
-          cmax = tr.cum_max[(it & 1) * BH + bh] + step;
-        }
+        if (prev_changed)
+          cmax = tr.cum_max[(it & 1) * BH + bh] + wave_top(lane < K ? tr.delta[bh * K + lane] : 0.0f);
         if (s_in == 0 && threadIdx.x == 0) tr.cum_max[((it + 1) & 1) * BH + bh] = cmax;
         __syncthreads();
       }
@@ -307,48 +390,74 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
     const int n = static_cast<int>(S - base < ns * kSlab ? S - base : ns * kSlab);
     int32_t* const lab = labels + bh * S + base;
     int nl = n;  // tokens to assign
+    __syncthreads();  // every wave is done with the previous lists
+    if (threadIdx.x == 0) { nlist_s = 0; npend_s = 0; }
+    __syncthreads();
     if (filter) {
-      __syncthreads();  // every wave is done with the previous list
-      if (threadIdx.x == 0) nlist_s = 0;
-      __syncthreads();
       const float c = 1.001f * sqrtf(c2max);
-      for (int i0 = 0; i0 < n; i0 += kAsgThreads) {
-        const int i = i0 + static_cast<int>(threadIdx.x);
-        const bool need = i < n && !bounds_hold(tr.ul[bh * S + base + i], cum_s[lab[i]], cmax, c);
-        const uint64_t m = __ballot(need);
-        int at = 0;
-        if (lane == 0 && m) at = atomicAdd(&nlist_s, __popcll(m));
-        at = __builtin_amdgcn_readfirstlane(at);
-        if (need) list_s[at + __popcll(m & lt_mask)] = i;
+      const float2* ul = tr.ul + bh * S + base;
+      // kLd tokens' loads in flight per thread
+      constexpr int kLd = 4;
+      for (int i0 = 0; i0 < n; i0 += kLd * kAsgThreads) {
+        float2 st[kLd];
+        int lb[kLd];
+#pragma unroll
+        for (int q = 0; q < kLd; ++q) {
+          int i = i0 + q * kAsgThreads + static_cast<int>(threadIdx.x);
+          i = i < n ? i : n - 1;
+          st[q] = ul[i];
+          lb[q] = lab[i];
+        }
+#pragma unroll
+        for (int q = 0; q < kLd; ++q) {
+          const int i = i0 + q * kAsgThreads + static_cast<int>(threadIdx.x);
+          const bool need = i < n && !bounds_hold(st[q], cum_s[lb[q]], cmax, c);
+          const uint64_t m = __ballot(need);
+          int at = 0;
+          if (lane == 0 && m) at = atomicAdd(&nlist_s, __popcll(m));
+          at = __builtin_amdgcn_readfirstlane(at);
+          if (need) list_s[at + __popcll(m & lt_mask)] = static_cast<uint16_t>(i);
+        }
       }
       __syncthreads();
       nl = nlist_s;
     }
     const int64_t b = bh / H, h = bh - b * H;
     const int64_t xseg = ((b * S + base) * H + h) * D;
-    for (int p0 = wave * 32; p0 < nl; p0 += 32 * kAsgWaves) {
+    // token operands: lane (li, g) holds dimensions 16 ks + 8 g + [0, 8) of its
+    // token.  The next step's are loaded once this step's MFMAs have read them;
+    // tokens that are split (fp16, fp32) GK k-steps at a time as they are used,
+    // to stay under 128 registers.
+    constexpr bool AHEAD = !XSPLIT;
+    constexpr int GK = AHEAD ? NKS : DT == kF16 || MB == 1 ? NKS / 2 : 2;
+    Raw8<DT> raw[GK];
+    auto token_of = [&](int p0) -> int {
+      const int p = p0 + li < nl ? p0 + li : nl - 1;  // lanes past the end repeat the last token
+      return filter ? list_s[p] : p;
+    };
+    auto load_raw = [&](int i, int k0) {
+      const int64_t x0 = xseg + static_cast<int64_t>(i) * H * D;
+#pragma unroll
+      for (int q = 0; q < GK; ++q) raw[q].load(x, x0 + 16 * (k0 + q) + 8 * g);
+    };
+    bool moved = false;
+    int p0 = wave * 32;
+    int i = p0 < nl ? token_of(p0) : 0;
+    if (AHEAD && p0 < nl) load_raw(i, 0);
+    while (p0 < nl) {
       // the centroid operands are read from LDS in every step: kept in registers
       // across steps they do not fit
       asm volatile("" ::: "memory");
       const bool valid = p0 + li < nl;
-      const int p = valid ? p0 + li : nl - 1;  // lanes past the end repeat the last token
-      const int i = filter ? list_s[p] : p;
-      const int64_t x0 = xseg + static_cast<int64_t>(i) * H * D;
       float xx = 0.0f;
       v16f a[MB];
 #pragma unroll
       for (int m = 0; m < MB; ++m)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) a[m][r] = -0.5f * lds.cn[32 * m + 8 * (r >> 2) + 4 * g + (r & 3)];
-      // token operands: lane (li, g) holds dimensions 16 ks + 8 g + [0, 8) of its
-      // token, GK k-steps' loads in flight (all; two with fp32 tokens and 64
-      // centroids, to stay under 128 registers)
-      constexpr int GK = DT == kF32 && MB == 2 ? 2 : NKS;
+        for (int r = 0; r < 16; ++r) a[m][r] = lds.a0[32 * m + 8 * (r >> 2) + 4 * g + (r & 3)];
 #pragma unroll 1
       for (int k0 = 0; k0 < NKS; k0 += GK) {
-        Raw8<DT> raw[GK];
-#pragma unroll
-        for (int q = 0; q < GK; ++q) raw[q].load(x, x0 + 16 * (k0 + q) + 8 * g);
+        if constexpr (!AHEAD) load_raw(i, k0);
 #pragma unroll
         for (int q = 0; q < GK; ++q) {
           const int ks = k0 + q;
@@ -376,67 +485,116 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
             if constexpr (XSPLIT) a[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xl, a[m], 0, 0, 0);
           }
         }
+        if constexpr (AHEAD) {
+          // operand reads kAheadLds MFMAs ahead of their use: read as late as the
+          // register allocator likes, every MFMA waited for its LDS latency
+          constexpr int kAheadLds = 3;
+          __builtin_amdgcn_sched_group_barrier(0x100, 4 * MB + kAheadLds, 0);
+#pragma unroll
+          for (int q = 0; q < 2 * MB * GK; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+        }
       }
-      xx += __shfl_xor(xx, 32, 64);
+      const int p_next = p0 + 32 * kAsgWaves;
+      const int i_next = token_of(p_next);  // past the end: the last token again, unused
+      if constexpr (AHEAD) load_raw(i_next, 0);
+      xx += from_pair(xx, g);
       // X C and C^2 from above: 2^-110 covers squares lost to underflow, 1.001 the roundings of the norms
-      const float xc = sqrtf((xx + 0x1p-110f) * (c2max + 0x1p-110f));
+      const float xc = __builtin_amdgcn_sqrtf((xx + 0x1p-110f) * (c2max + 0x1p-110f));
       const float gap = 1.001f * (kGapXC * xc + kGapCC * c2max) + 0x1p-120f;
-      float top = -INFINITY;
-#pragma unroll
-      for (int m = 0; m < MB; ++m)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) top = fmaxf(top, a[m][r]);
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
-      const float thr = top - gap;
-      int cnt = 0, bj = 0;
-      float second = -INFINITY;  // the largest a_j of the others, where one centroid is near
+      const bool finite = gap < INFINITY;  // then every a_j is
+      // the two largest, each with its centroid's row in the last six bits
+      float top = -INFINITY, second = -INFINITY;
 #pragma unroll
       for (int m = 0; m < MB; ++m)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const bool near = !(a[m][r] < thr);  // NaN on either side counts as near
-          cnt += near ? 1 : 0;
-          bj = near ? 32 * m + 8 * (r >> 2) + (r & 3) : bj;
-          second = near ? second : fmaxf(second, a[m][r]);
+          const float v = __uint_as_float((__float_as_uint(a[m][r]) & ~63u) | (32 * m + 8 * (r >> 2) + (r & 3)));
+          second = __builtin_amdgcn_fmed3f(top, second, v);
+          top = vmax(top, v);
         }
-      bj = cnt ? bj + 4 * g : 0;
-      const int cnt2 = cnt + __shfl_xor(cnt, 32, 64);
-      bj = max(bj, __shfl_xor(bj, 32, 64));  // the one near centroid, if there is one
-      second = fmaxf(second, __shfl_xor(second, 32, 64));
-      // unsettled tokens, two at a time with up to 32 centroids
-      const bool unsettled = cnt2 != 1;
-      uint32_t open = static_cast<uint32_t>(__ballot(unsettled && valid));
-      while (open) {
-        const int i0 = __builtin_ctz(open);
+      top = __uint_as_float(__float_as_uint(top) | 4 * g);
+      const float top_o = from_pair(top, g), second_o = from_pair(second, g);
+      second = vmax(fminf(top, top_o), vmax(second, second_o));
+      top = vmax(top, top_o);
+      const bool settled = finite && top - second > gap;
+      int bj = __float_as_uint(top) & 63;
+      int cnt = 1, j0 = 0, j1 = 0;  // near centroids, the first and the last of them
+      if (__any(!settled)) {
+        const float thr = top - gap;
+        uint32_t near_m = 0u;  // bit 16 m + r: centroid 32 m + 8 (r / 4) + 4 g + r % 4 is near
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) near_m |= !(a[m][r] < thr) ? 1u << (16 * m + r) : 0u;
+        auto row_of = [&](int bit) -> int { return 2 * (bit & ~3) + (bit & 3) + 4 * g; };
+        const int lo = near_m ? row_of(__builtin_ctz(near_m)) : 64, hi = near_m ? row_of(31 - __builtin_clz(near_m)) : 0;
+        j0 = min(lo, static_cast<int>(from_pair(static_cast<uint32_t>(lo), g)));
+        j1 = max(hi, static_cast<int>(from_pair(static_cast<uint32_t>(hi), g)));
+        const uint32_t n = __popc(near_m);
+        cnt = settled ? 1 : static_cast<int>(n + from_pair(n, g));
+        // one near (the numbers in the last bits can hide that), or all are suspect: the full settle
+        if (!settled && (cnt < 2 || !finite)) cnt = 64;
+      }
+      uint32_t open = static_cast<uint32_t>(__ballot(cnt > 2 && valid));
+      while (open) {  // two tokens at a time with up to 32 centroids
+        const int t0 = __builtin_ctz(open);
         open &= open - 1;
-        int i1 = i0;
+        int t1 = t0;
         if (MB == 1 && open) {
-          i1 = __builtin_ctz(open);
+          t1 = __builtin_ctz(open);
           open &= open - 1;
         }
-        const int ti = __shfl(i, MB == 1 && lane >= 32 ? i1 : i0, 64);
+        const int ti = __shfl(i, MB == 1 && lane >= 32 ? t1 : t0, 64);
         const int le = assign_exact<D, DT, MB>(lds, x, xseg + static_cast<int64_t>(ti) * H * D, lane);
         const int l0 = __builtin_amdgcn_readlane(le, 0), l1 = __builtin_amdgcn_readlane(le, 32);
-        if (li == i0) bj = l0;
-        else if (li == i1) bj = l1;
+        if (li == t0) bj = l0;
+        else if (li == t1) bj = l1;
       }
-      if (lane < 32 && valid) {
+      const bool pair = cnt == 2 && valid && lane < 32;
+      const uint64_t pm = __ballot(pair);
+      if (pm) {
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&npend_s, __popcll(pm));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (pair) pend_s[at + __popcll(pm & lt_mask)] = static_cast<uint32_t>(i | j0 << 16 | j1 << 24);
+      }
+      if (lane < 32 && valid && cnt != 2) {
         const int32_t old = prev_changed ? lab[i] : -1;
         lab[i] = bj;
-        if (__any(old != bj) && lane == 0) changed[bh] = 1;
-        if (tr.ul) {
-          // |x - c_j|^2 = |x|^2 - 2 a_j, with twice the error of a_j (and that of
-          // the stored norms) below the gap and that of |x|^2 below 2^-15 of it
-          const float e = gap + 0x1p-15f * xx;
-          float2 st = make_float2(INFINITY, 0.0f);  // never holds
-          if (!unsettled) {
-            st.x = sqrtf(fmaxf(xx - 2.0f * top, 0.0f) + e) * (1.0f + kOut) - cum_s[bj];
-            st.y = sqrtf(fmaxf(xx - 2.0f * second - e, 0.0f)) * (1.0f - kOut) + cmax;
-          }
-          tr.ul[bh * S + base + i] = st;
+        moved |= old != bj;
+      }
+      if (tr.ul && lane < 32 && valid) {
+        // |x - c_j|^2 = |x|^2 - 2 a_j, with twice the error of a_j (and that of
+        // the stored norms) below the gap and that of |x|^2 below 2^-15 of it
+        const float e = gap + 0x1p-15f * xx;
+        float2 st = make_float2(INFINITY, 0.0f);  // never holds
+        if (settled) {
+          st.x = __builtin_amdgcn_sqrtf(fmaxf(xx - 2.0f * top, 0.0f) + e) * (1.0f + kOut) - cum_s[bj];
+          st.y = __builtin_amdgcn_sqrtf(fmaxf(xx - 2.0f * second - e, 0.0f)) * (1.0f - kOut) + cmax;
         }
+        tr.ul[bh * S + base + i] = st;
+      }
+      p0 = p_next;
+      i = i_next;
+    }
+    __syncthreads();
+    const int np = npend_s;
+    for (int q0 = wave * 32; q0 < np; q0 += 32 * kAsgWaves) {
+      const bool valid = q0 + li < np;
+      const uint32_t e = pend_s[valid ? q0 + li : np - 1];
+      const int t = e & 0xffff;
+      const int bj = assign_pair<D, DT, MB>(lds, x, xseg + static_cast<int64_t>(t) * H * D, e >> (16 + 8 * g) & 0xff);
+      if (valid && g == 0) {
+        const int32_t old = prev_changed ? lab[t] : -1;
+        lab[t] = bj;
+        moved |= old != bj;
       }
     }
+    // one store per wave and segment: all slices' flags share a few cache lines
+    if (__any(moved) && lane == 0) changed[bh] = 1;
   }
 }
 
@@ -457,9 +615,10 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
 // from the one the partial sums stand for -- the same bits as summing anew --
 // unless more than a quarter of the chunk moved.
 //
-// Bound by the row reads (and the LDS sort ahead of them); with one column and
-// a 2-byte load per lane the full sums took 132 us a round at
-// 40 x 32768 x 128 bf16, 32 clusters (2.5 TB/s).
+// Bound by the row reads and the LDS sort ahead of them: at 40 x 32768 x 128
+// bf16 with 32 clusters the first round (the ranges included) takes 125 us, the
+// later ones 67, 31, 18, then 14 as fewer tokens move (every round 132 us with
+// one column and a 2-byte load per lane and no moves).
 constexpr int kUpdThreads = 512;
 constexpr int kMaxMoved = kChunk / 4;
 
@@ -479,7 +638,7 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
   __shared__ int running[kMaxKAssign];
   __shared__ int net_s[kMaxKAssign];
   __shared__ int wcnt[NW][kMaxKAssign];
-  __shared__ uint32_t range_s[2];  // largest magnitude; smallest nonzero one, minus 1 (fp32 bits)
+  __shared__ uint32_t range_s[2];  // largest magnitude; smallest nonzero one, minus 1 (bits)
   const int64_t nchunk = (S + kChunk - 1) / kChunk;
   const int64_t bh = blockIdx.x / nchunk, c = blockIdx.x % nchunk;
   if (changed[bh] == 0) return;  // converged slice (uniform per workgroup)
@@ -622,7 +781,7 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     if (tr.ul) tr.touched[bh * K + tid] = 1;
   }
   // column sums over the sorted runs of this group's clusters
-  uint32_t big = 0u, small = 0xffffffffu;
+  typename Raw8<DT>::Mag big = 0, small = ~big;
   for (int j = g; j < K; j += NG) {
     const int p1 = start_s[j + 1];
     double acc[8];
@@ -642,14 +801,7 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
           raw[i].to_f32(v);
 #pragma unroll
           for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(v[k]);
-          if (first) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-              const uint32_t a = __float_as_uint(v[k]) & 0x7fffffffu;
-              big = a > big ? a : big;
-              small = a - 1u < small ? a - 1u : small;  // 0 - 1 wraps to the top
-            }
-          }
+          if (first) raw[i].range(big, small);
         }
       }
     }
@@ -658,17 +810,17 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     for (int k = 0; k < 4; ++k) o[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
   }
   if (tr.ul && first) {
-    atomicMax(&range_s[0], big);
-    atomicMin(&range_s[1], small);
+    atomicMax(&range_s[0], Raw8<DT>::widest(big, true));
+    atomicMin(&range_s[1], Raw8<DT>::widest(small, false));
     __syncthreads();
     if (tid == 0) {
-      // mantissa bits below the leading one of a value of this dtype
-      constexpr int kMant = DT == kF32 ? 23 : DT == kF16 ? 10 : 7;
-      const int eb = static_cast<int>(range_s[0] >> 23);  // biased exponents
-      int es = static_cast<int>((range_s[1] + 1u) >> 23);
+      constexpr int kMant = DT == kF32 ? 23 : DT == kF16 ? 10 : 7;  // mantissa bits below the leading one
+      constexpr int kExpTop = DT == kF16 ? 31 : 255;                // of infinities and NaNs
+      const int eb = static_cast<int>(range_s[0] >> kMant);         // biased exponents
+      int es = static_cast<int>((range_s[1] + 1u) >> kMant);
       es = es < 1 ? 1 : es;
       // 2^(eb + 1) * 2^12 terms over a last bit of 2^(es - kMant): 53 bits hold them
-      tr.exact[bh * nchunk + c] = eb < 255 && (range_s[0] == 0u || eb + 1 + 12 - (es - kMant) <= 53) ? 1 : 0;
+      tr.exact[bh * nchunk + c] = eb < kExpTop && (range_s[0] == 0u || eb + 1 + 12 - (es - kMant) <= 53) ? 1 : 0;
     }
   }
 }
