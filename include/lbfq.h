@@ -367,6 +367,23 @@ typedef struct {
 
 int lbfq_blasst_attend(const lbfq_blasst_attend_params* p, lbfq_stream_t stream);
 
+/* The simulator with bf16 matmul operands, on the matrix cores (the same
+ * statistics and rungs as the fp32 entries above, P rounded to bf16 before PV).
+ * operand: x (S, H, D) of dtype `dtype` rounded to bf16, or with `quantise`
+ * fake-quantised per head first (as lbfq_head_fp8_quant, whose amax_ws, counts,
+ * sqerr and optional scale it takes), to out as (H, S, D) rows or, transposed,
+ * (H, D, S).  scan / attend: q and k as rows, v transposed, sm_scale > 0;
+ * attend's mode, keep, dropped and P statistics as in
+ * lbfq_blasst_attend_params.  S % 128 == 0, D in {64, 128}, H <= 256 with quantise. */
+int lbfq_blasst_operand_bf16(const void* x, int dtype, int64_t S, int64_t H, int64_t D, int quantise, int transposed,
+                             uint16_t* out, float* scale, uint32_t* amax_ws, int64_t* counts, double* sqerr,
+                             lbfq_stream_t stream);
+int lbfq_blasst_scan_bf16(const uint16_t* q, const uint16_t* k, int64_t S, int64_t H, int64_t D, float sm_scale,
+                          float* final_max, uint32_t* tile_margin, uint32_t* tile_bmax, lbfq_stream_t stream);
+int lbfq_blasst_attend_bf16(const uint16_t* q, const uint16_t* k, const uint16_t* v_t, int64_t S, int64_t H, int64_t D,
+                            float sm_scale, int mode, const float* final_max, const uint8_t* keep, float* out,
+                            float* dropped, int64_t* p_counts, double* p_sqerr, lbfq_stream_t stream);
+
 /* ---- measurement probe ----------------------------------------------------- */
 /* HBM streaming probe (no counterpart in the reference: it measures the
  * ceiling the prepass is held against).  mode 0 reads `bytes` from src

@@ -172,6 +172,10 @@ _SIGS = {
     "lbfq_head_fp8_quant": (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp]),
     "lbfq_blasst_scan": (_i32, [_vp, _vp, _i64, _i64, _i64, _f32, _vp, _vp, _vp, _vp]),
     "lbfq_blasst_keep": (_i32, [_vp, _vp, _i64, _i64, _vp, _i32, _vp, _vp, _vp]),
+    "lbfq_blasst_operand_bf16": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "lbfq_blasst_scan_bf16": (_i32, [_vp, _vp, _i64, _i64, _i64, _f32, _vp, _vp, _vp, _vp]),
+    "lbfq_blasst_attend_bf16": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _f32, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
+                                       _vp]),
     "lbfq_blasst_attend": (_i32, [ctypes.POINTER(BlasstAttendParams), _vp]),
     "lbfq_sdpa_dequant": (_i32, [ctypes.POINTER(SdpaDequantParams), _vp]),
     "lbfq_sdpa_fwd": (_i32, [ctypes.POINTER(SdpaParams), _vp]),

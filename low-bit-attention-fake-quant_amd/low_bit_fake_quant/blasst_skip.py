@@ -13,7 +13,9 @@ of block maxima (a skipped block never raises it); a tile that keeps no block
 keeps its block of largest max (``blasst_skip.py:348-386, 584-619``).
 
 ``simulate_workload`` runs on four HIP kernels (``lbfq_head_fp8_quant``,
-``lbfq_blasst_scan``, ``lbfq_blasst_keep``, ``lbfq_blasst_attend``): a scan
+``lbfq_blasst_scan``, ``lbfq_blasst_keep``, ``lbfq_blasst_attend``; with bf16
+matmul operands their matrix-core counterparts ``lbfq_blasst_operand_bf16``,
+``lbfq_blasst_scan_bf16`` and ``lbfq_blasst_attend_bf16``): a scan
 pass forms the scores once per row and records row maxima and per-tile
 margins, a keep pass turns the margins into masks, and one attend pass per
 rung (per threshold for the skip rung) accumulates the output.  The tile
@@ -333,6 +335,53 @@ class _Sim:
         return out, drop, pc, pe
 
 
+class _SimBf16(_Sim):
+    """The same over bf16 operands on the matrix cores: q and k as (H, S, D)
+    rows, v as (H, D, S)."""
+
+    def operand(self, x3, *, quantise: bool, transposed: bool):
+        """(operand, QuantStats or None) of an (S, H, D) tensor."""
+        x3 = x3.contiguous()
+        if x3.dtype not in _lib.DTYPE_CODE:
+            raise TypeError(f"unsupported dtype {x3.dtype}")
+        s, h, d = self.s, self.h, self.d
+        out = torch.empty((h, d, s) if transposed else (h, s, d), dtype=torch.bfloat16, device=self.dev)
+        ws = counts = sqerr = None
+        if quantise:
+            ws = torch.empty(h, dtype=torch.int32, device=self.dev)
+            counts = torch.zeros(2, dtype=torch.int64, device=self.dev)
+            sqerr = torch.zeros(1, dtype=torch.float64, device=self.dev)
+        _lib.check(self.lib.lbfq_blasst_operand_bf16(
+            x3.data_ptr(), _lib.DTYPE_CODE[x3.dtype], s, h, d, int(quantise), int(transposed), out.data_ptr(), None,
+            _lib.ptr(ws), _lib.ptr(counts), _lib.ptr(sqerr), self.stream), "blasst_operand_bf16")
+        if not quantise:
+            return out, None
+        n = x3.numel()
+        c = counts.tolist()
+        return out, QuantStats(c[0] / n, c[1] / n, math.sqrt(float(sqerr.item()) / n))
+
+    def scan(self, q, k):
+        fm = torch.empty(self.h, self.s, dtype=torch.float32, device=self.dev)
+        n = self.h * self.nb * self.nb
+        tm = torch.empty(n, dtype=torch.int32, device=self.dev)
+        tb = torch.empty(n, dtype=torch.int32, device=self.dev)
+        _lib.check(self.lib.lbfq_blasst_scan_bf16(q.data_ptr(), k.data_ptr(), self.s, self.h, self.d, self.sm,
+                                                  fm.data_ptr(), tm.data_ptr(), tb.data_ptr(), self.stream),
+                   "blasst_scan_bf16")
+        return fm, tm, tb
+
+    def attend(self, q, k, v, fm, mode, round_p, keep=None, dropped=False, p_stats=False):
+        out = torch.empty(self.s, self.h, self.d, dtype=torch.float32, device=self.dev)
+        drop = torch.empty(self.h, self.s, dtype=torch.float32, device=self.dev) if dropped else None
+        pc = torch.zeros(2, dtype=torch.int64, device=self.dev) if p_stats else None
+        pe = torch.zeros(1, dtype=torch.float64, device=self.dev) if p_stats else None
+        _lib.check(self.lib.lbfq_blasst_attend_bf16(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), self.s, self.h, self.d, self.sm, mode, fm.data_ptr(),
+            _lib.ptr(keep), out.data_ptr(), _lib.ptr(drop), _lib.ptr(pc), _lib.ptr(pe), self.stream),
+            "blasst_attend_bf16")
+        return out, drop, pc, pe
+
+
 def _quantiles(dm: torch.Tensor):
     sd = dm.float().flatten().sort().values
     n = sd.numel()
@@ -365,12 +414,17 @@ def simulate_workload(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, skip
     want_fp8 = any(lv in levels for lv in (LEVEL_FP8_QKV, LEVEL_FP8_STATIC_P, LEVEL_FP8_SKIP))
     round_p = matmul_dtype == torch.bfloat16
     dev = q.device
-    sim = _Sim(s, h, d, 1.0 / math.sqrt(d), dev)
+    on_mfma = matmul_dtype == torch.bfloat16
+    sim = (_SimBf16 if on_mfma else _Sim)(s, h, d, 1.0 / math.sqrt(d), dev)
     torch.cuda.reset_peak_memory_stats(dev)
     result = SimulationResult()
 
     if LEVEL_REFERENCE in levels:
-        qr, kr, vr = (t[0].to(matmul_dtype).float().contiguous() for t in (q, k, v))
+        if on_mfma:
+            qr, kr, vr = (sim.operand(t[0], quantise=False, transposed=tr)[0]
+                          for t, tr in ((q, False), (k, False), (v, True)))
+        else:
+            qr, kr, vr = (t[0].to(matmul_dtype).float().contiguous() for t in (q, k, v))
         fm, _, _ = sim.scan(qr, kr)
         out, *_ = sim.attend(qr, kr, vr, fm, 0, round_p)
         result.outputs[LEVEL_REFERENCE] = out.view(1, s, h, d)
@@ -379,7 +433,10 @@ def simulate_workload(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, skip
     if want_fp8:
         qd, kd, vd = [], [], []
         for name, t, dst in (("q", q, qd), ("k", k, kd), ("v", v, vd)):
-            _, mm, _, st = _head_quant(t[0], matmul_dtype, False)
+            if on_mfma:
+                mm, st = sim.operand(t[0], quantise=True, transposed=name == "v")
+            else:
+                _, mm, _, st = _head_quant(t[0], matmul_dtype, False)
             dst.append(mm)
             result.quant_stats[name] = st
         qd, kd, vd = qd[0], kd[0], vd[0]

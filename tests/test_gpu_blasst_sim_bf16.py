@@ -1,0 +1,57 @@
+"""The simulator's matrix-core kernels (bf16 matmul operands) at the edges of
+their work split: one key block, a workgroup whose second query tile lies past
+S, every input dtype, both head sizes, and operands that share one tensor."""
+
+import pytest
+import torch
+
+from conftest import cpu_randn
+from oracle import blasst_sim as osim
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(a, b):
+    """As tests/test_gpu_blasst_sim.py: a P weight may cross a bf16 or E4M3
+    rounding boundary (one step is 2^-8 of the weight at most)."""
+    a, b = a.double().flatten(), b.double().flatten()
+    assert float(a @ b / (a.norm() * b.norm())) >= 0.99999
+    assert float((a - b).abs().max()) <= 2e-3 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("s,h,d,dtype", [(128, 3, 64, torch.bfloat16), (128, 1, 128, torch.float32),
+                                         (256, 2, 128, torch.float16), (384, 5, 64, torch.float32),
+                                         (640, 1, 128, torch.bfloat16)])
+def test_rungs_match_oracle(gpu, s, h, d, dtype):
+    from low_bit_fake_quant import blasst_skip as bs
+    q, k, v = (cpu_randn(1, s, h, d, seed=90 + i, dtype=torch.float32) for i in range(3))
+    k[:, :128] *= 6.0          # the first block dominates: later ones can be skipped
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    ths = [0.05, 2.0]
+    res = bs.simulate_workload(q.to(gpu), k.to(gpu), v.to(gpu), skip_thresholds=ths)
+    ref = osim.simulate(q, k, v, skip_thresholds=ths, mm_dtype=torch.bfloat16)
+    for lv in ("bf16_ref", "fp8_qkv", "fp8_static_p"):
+        _close(res.outputs[lv][0].cpu(), ref[lv])
+    for th in ths:
+        _close(res.skip_outputs[th][0].cpu(), ref["skip"][th])
+        dg = res.skip_diagnostics[th]
+        assert dg.skip_rate == ref["skip_rate"][th] and dg.force_keep_count == ref["force"][th]
+        assert abs(dg.dropped_mass_max - float(ref["dropped"][th].max())) < 1e-4
+    for name in ("q", "k", "v"):
+        st, so = res.quant_stats[name], ref["stats"][name]
+        assert st.saturation_rate == so["saturation_rate"] and st.underflow_zero_rate == so["underflow_zero_rate"]
+        assert abs(st.roundtrip_rmse - so["roundtrip_rmse"]) <= 1e-6 * so["roundtrip_rmse"] + 1e-12
+    sp, op = res.quant_stats["p"], ref["stats"]["p"]
+    assert abs(sp.underflow_zero_rate - op["underflow_zero_rate"]) < 1e-4
+    assert abs(sp.roundtrip_rmse - op["roundtrip_rmse"]) <= 1e-3 * op["roundtrip_rmse"]
+
+
+def test_one_tensor_as_all_three(gpu):
+    from low_bit_fake_quant import blasst_skip as bs
+    x = cpu_randn(1, 256, 2, 64, seed=4)
+    xg = x.to(gpu)
+    one = bs.simulate_workload(xg, xg, xg, skip_thresholds=[0.05])
+    three = bs.simulate_workload(xg, xg.clone(), xg.clone(), skip_thresholds=[0.05])
+    for lv in one.outputs:
+        assert torch.equal(one.outputs[lv], three.outputs[lv])
+    _close(one.outputs["bf16_ref"][0].cpu(), osim.simulate(x, x, x)["bf16_ref"])
