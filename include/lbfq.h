@@ -68,7 +68,7 @@ typedef struct {
   float had_scale;                         /* fp32(1/sqrt(D))                   */
   int quant_mode;                          /* LBFQ_Q_*                          */
   uint8_t* codes; int codes_layout;        /* LBFQ_LAYOUT_*                     */
-  int64_t codes_spitch;                    /* S extent of BHSD/BHDS buffers     */
+  int64_t codes_spitch;                    /* S extent of BHSD/BHDS buffers; rows [S, codes_spitch) get zero codes */
   float* scale;                            /* scale output (see strides)        */
   int64_t sc_b, sc_s, sc_h, sc_d;          /* element strides of scale          */
   uint32_t* amax_table;                    /* (B,H,D) fp32 bits, channel modes  */

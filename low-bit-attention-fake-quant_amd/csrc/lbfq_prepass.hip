@@ -14,6 +14,9 @@
 // hadamard.py:25-117, kmeans.py:84-89 / 127-135.
 #include <stdarg.h>
 
+#include <type_traits>
+
+
 #include "lbfq_common.h"
 #include "../../include/lbfq.h"
 
@@ -149,6 +152,27 @@ constexpr int kKeep = 4;        // resident passes per wave
 constexpr int kLB = 4;          // passes per wave in flight when streaming
 constexpr int kStageRows = 64;  // rows per BHDS staging chunk
 
+// Zero codes for the rows [S, pitch) of one (b, h): written by the workgroup of
+// its last tile, so that the buffer needs no clearing pass of its own.
+__device__ __forceinline__ void zero_padding(const RowTileArgs& a, int64_t bh, int tid) {
+  const int64_t pad = a.codes_spitch - a.S;
+  if (a.codes_layout == LBFQ_LAYOUT_BHSD) {
+    uint8_t* p = a.codes + (bh * a.codes_spitch + a.S) * a.D;  // D bytes a row: 16-byte pieces
+    for (int64_t e = tid; e < pad * (a.D / 16); e += kTileWaves * 64)
+      reinterpret_cast<uint4*>(p)[e] = make_uint4(0u, 0u, 0u, 0u);
+  } else if (a.codes_layout == LBFQ_LAYOUT_BHDS) {
+    uint8_t* p = a.codes + bh * a.D * a.codes_spitch + a.S;
+    const int64_t head = (4 - a.S % 4) % 4 < pad ? (4 - a.S % 4) % 4 : pad;  // bytes up to a word (the pitch is whole words)
+    const int64_t per = head + (pad - head) / 4;
+    for (int64_t e = tid; e < a.D * per; e += kTileWaves * 64) {
+      uint8_t* row = p + e / per * a.codes_spitch;
+      const int64_t i = e % per;
+      if (i < head) row[i] = 0;
+      else *reinterpret_cast<uint32_t*>(row + head + 4 * (i - head)) = 0u;
+    }
+  }
+}
+
 template <int DT, int QM, bool SUB, bool HAD>
 __global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a) {
   constexpr bool TILE_RED = QM == LBFQ_Q_FP8_BLOCK || QM == LBFQ_Q_MX_V || QM == LBFQ_Q_CHANNEL_AMAX;
@@ -207,6 +231,9 @@ __global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a)
       mfix[0] = m0.x; mfix[1] = m0.y; mfix[2] = m0.z; mfix[3] = m0.w;
       mfix[4] = m1.x; mfix[5] = m1.y; mfix[6] = m1.z; mfix[7] = m1.w;
     }
+  }
+  if constexpr (QM != LBFQ_Q_NONE && QM != LBFQ_Q_CHANNEL_AMAX) {
+    if (static_cast<uint32_t>(tile) + 1 == ntile && a.codes_spitch > a.S) zero_padding(a, bh, tid);
   }
   const bool sm0 = a.smoothed && a.smoothed_stage == 0, sm1 = a.smoothed && a.smoothed_stage == 1;
   __shared__ float red[kTileWaves][128];  // cross-wave reductions (D <= 128)
@@ -502,15 +529,26 @@ __global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a)
 // Sequential fp64 column sums of `chunk` rows (optionally gathered).
 // mode 0: write fp64 partial sums (B, nchunk, H, D);
 // mode 1: write fp32 means fp32(sum / rows_in_chunk) (B, nchunk, H, D).
-// One thread sums 8 adjacent columns of one (b, chunk, h) over the chunk's
-// rows in order; adjacent threads take adjacent 16-byte pieces of a row
-// (columns, then heads), so a wave reads contiguous memory.  Loads of 8 rows
-// are in flight before they are added, in row order.
-template <int DT>
+// One thread sums NC adjacent columns of one (b, chunk, h) over the chunk's
+// rows in order; adjacent threads take adjacent columns, then heads, so a wave
+// reads contiguous memory.  The order leaves one serial chain per column, so
+// latency bounds a small problem and the mix of rows in flight a large one:
+// ROWS rows of loads are in flight before they are added, a gather's next
+// indices with them.  Measured on bf16 in 256-row chunks, us (NC, ROWS):
+//                             8, 8   8, 16   4, 16   2, 16   2, 32   2, 64
+//   4 x 1000 x 64               28      26      20      16      15      16
+//   12 x 8192 x 128             44      35      26      23      18      17
+//   12 x 32768 x 128            58      46      34      31      26      26
+//   40 x 32768 x 128            74      69      63      61      62      68
+//   40 x 75776 x 128           136     139     139     139     141     147
+// hence (2, 32).  Gathered rows, each 256 bytes apart from the next anyway,
+// prefer wide pieces once those make four waves per CU: 40 x 32768 x 128
+// gathered takes 172 at (8, 8), 70 at (2, 32) and 67 at (8, 32).
+template <int DT, bool GATHER, int NC, int ROWS>
 __global__ void __launch_bounds__(256) colsum_kernel(const void* x, int64_t B, int64_t S, int64_t H, int64_t D,
-                                                     int chunk, const int32_t* gather, int mode, double* part,
-                                                     float* mean) {
-  const int64_t ndg = D / 8;
+                                                    int chunk, const int32_t* gather, int mode, double* part,
+                                                    float* mean) {
+  const int64_t ndg = D / NC;
   const int64_t nchunk = (S + chunk - 1) / chunk;
   int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= B * nchunk * H * ndg) return;
@@ -519,48 +557,77 @@ __global__ void __launch_bounds__(256) colsum_kernel(const void* x, int64_t B, i
   const int64_t c = t % nchunk;
   const int64_t b = t / nchunk;
   const int64_t s0 = c * chunk;
-  const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
-  const int64_t d0 = dg * 8;
-  double acc[8];
+  const int n = static_cast<int>(s0 + chunk < S ? chunk : S - s0);
+  const int64_t d0 = dg * NC;
+  constexpr int ES = DT == kF32 ? 4 : 2, NW = NC * ES / 4;  // words of a row piece
+  struct __attribute__((aligned(NW >= 4 ? 16 : 4 * NW))) Raw {
+    uint32_t w[NW];
+  };
+  const uint8_t* xc = static_cast<const uint8_t*>(x) + ((b * S * H + h) * D + d0) * ES;
+  const int64_t pitch = H * D * ES;
+  const int32_t* gp = GATHER ? gather + (b * H + h) * S + s0 : nullptr;
+  double acc[NC];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = 0.0;
-  constexpr int kRows = 8;
-  for (int64_t sb = s0; sb < s1; sb += kRows) {
-    float v[kRows][8];
+  for (int k = 0; k < NC; ++k) acc[k] = 0.0;
+  // a row past the chunk's end reads its first one (and is not added)
+  int32_t idx[GATHER ? ROWS : 1];
+  auto fetch = [&](int r0) {
+    if constexpr (GATHER) {
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-      int64_t s = sb + i < s1 ? sb + i : s0;  // a safe row past the chunk end (not added)
-      if (gather) s = gather[(b * H + h) * S + s];
-      load8t<DT>(x, ((b * S + s) * H + h) * D + d0, v[i]);
+      for (int i = 0; i < ROWS; ++i) idx[i] = gp[r0 + i < n ? r0 + i : 0];
     }
+  };
+  fetch(0);
+  for (int r0 = 0; r0 < n; r0 += ROWS) {
+    Raw raw[ROWS];
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-      if (sb + i < s1) {
+    for (int i = 0; i < ROWS; ++i) {
+      const int64_t s = GATHER ? idx[i] : s0 + (r0 + i < n ? r0 + i : 0);
+      raw[i] = *reinterpret_cast<const Raw*>(xc + s * pitch);
+    }
+    if (r0 + ROWS < n) fetch(r0 + ROWS);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(v[i][k]);
+    for (int i = 0; i < ROWS; ++i) {
+      if (r0 + i < n) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+          float v;
+          if constexpr (DT == kF32) v = __uint_as_float(raw[i].w[k]);
+          else if constexpr (DT == kBF16) v = bf16_bits_to_f32(static_cast<uint16_t>(raw[i].w[k / 2] >> (16 * (k & 1))));
+          else v = f16_bits_to_f32(static_cast<uint16_t>(raw[i].w[k / 2] >> (16 * (k & 1))));
+          acc[k] += static_cast<double>(v);
+        }
       }
     }
   }
   const int64_t o = ((b * nchunk + c) * H + h) * D + d0;
-  if (mode == 0) {
+  const double cnt = static_cast<double>(n);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) part[o + k] = acc[k];
-  } else {
-    const double n = static_cast<double>(s1 - s0);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) mean[o + k] = static_cast<float>(acc[k] / n);
+  for (int k = 0; k < NC; ++k) {
+    if (mode == 0) part[o + k] = acc[k];
+    else mean[o + k] = static_cast<float>(acc[k] / cnt);
   }
 }
 
-// Sum the chunk partials in chunk order; mean = fp32(total / S).
+// Sum the chunk partials in chunk order; mean = fp32(total / S).  32 partials
+// of a column are in flight before they are added.
 __global__ void colsum_finalize_kernel(const double* part, int64_t B, int64_t nchunk, int64_t H, int64_t D,
                                        int64_t S, float* mean) {
   int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= B * H * D) return;
-  int64_t d = i % D, h = (i / D) % H, b = i / (D * H);
+  const int64_t hd = i % (H * D), b = i / (D * H);
+  const double* p = part + b * nchunk * H * D + hd;
   double t = 0.0;
-  for (int64_t c = 0; c < nchunk; ++c) t += part[((b * nchunk + c) * H + h) * D + d];
-  mean[(b * H + h) * D + d] = static_cast<float>(t / static_cast<double>(S));
+  constexpr int kAhead = 32;
+  for (int64_t c0 = 0; c0 < nchunk; c0 += kAhead) {
+    double v[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) v[k] = p[(c0 + k < nchunk ? c0 + k : nchunk - 1) * H * D];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      if (c0 + k < nchunk) t += v[k];
+  }
+  mean[i] = static_cast<float>(t / static_cast<double>(S));
 }
 
 __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v) {
@@ -687,15 +754,25 @@ extern "C" int lbfq_colsum(const void* x, int dtype, int64_t B, int64_t S, int64
   LBFQ_CHECK_ARG(mode == 0 ? partial != nullptr : mean != nullptr, "lbfq_colsum: missing output");
   LBFQ_CHECK_ARG(dtype >= 0 && dtype <= 2, "lbfq_colsum: bad dtype %d", dtype);
   const int64_t nchunk = (S + chunk - 1) / chunk;
-  const int64_t nthreads = B * nchunk * H * (D / 8);
-  const dim3 grid(static_cast<unsigned>((nthreads + 255) / 256)), block(256);
+  const bool wide = gather && B * nchunk * H * (D / 8) >= 4 * 256 * 64;
+  const int64_t nthreads = B * nchunk * H * (D / (wide ? 8 : 2));
+  const unsigned nt = wide ? 64 : 256;
+  const dim3 grid(static_cast<unsigned>((nthreads + nt - 1) / nt)), block(nt);
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == kBF16)
-    hipLaunchKernelGGL(colsum_kernel<kBF16>, grid, block, 0, st, x, B, S, H, D, chunk, gather, mode, partial, mean);
-  else if (dtype == kF16)
-    hipLaunchKernelGGL(colsum_kernel<kF16>, grid, block, 0, st, x, B, S, H, D, chunk, gather, mode, partial, mean);
-  else
-    hipLaunchKernelGGL(colsum_kernel<kF32>, grid, block, 0, st, x, B, S, H, D, chunk, gather, mode, partial, mean);
+#define LBFQ_CS(DT, GA, NC, ROWS)                                                                                \
+  hipLaunchKernelGGL((colsum_kernel<DT, GA, NC, ROWS>), grid, block, 0, st, x, B, S, H, D, chunk, gather, mode, \
+                     partial, mean)
+#define LBFQ_CS_DT(DT)                                    \
+  do {                                                    \
+    if (wide) LBFQ_CS(DT, true, 8, (DT == kF32 ? 16 : 32)); \
+    else if (gather) LBFQ_CS(DT, true, 2, 32);            \
+    else LBFQ_CS(DT, false, 2, 32);                       \
+  } while (0)
+  if (dtype == kBF16) LBFQ_CS_DT(kBF16);
+  else if (dtype == kF16) LBFQ_CS_DT(kF16);
+  else LBFQ_CS_DT(kF32);
+#undef LBFQ_CS_DT
+#undef LBFQ_CS
   LBFQ_LAUNCH_CHECK("lbfq_colsum");
   return 0;
 }
@@ -704,7 +781,7 @@ extern "C" int lbfq_colsum_finalize(const double* partial, int64_t B, int64_t nc
                                     int64_t S, float* mean, lbfq_stream_t stream) {
   LBFQ_CHECK_ARG(partial && mean && nchunk > 0 && S > 0, "lbfq_colsum_finalize: bad args");
   int64_t n = B * H * D;
-  hipLaunchKernelGGL(colsum_finalize_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
+  hipLaunchKernelGGL(colsum_finalize_kernel, dim3(static_cast<unsigned>((n + 63) / 64)), dim3(64), 0,
                      static_cast<hipStream_t>(stream), partial, B, nchunk, H, D, S, mean);
   LBFQ_LAUNCH_CHECK("lbfq_colsum_finalize");
   return 0;

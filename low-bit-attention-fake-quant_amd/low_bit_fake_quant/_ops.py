@@ -91,16 +91,22 @@ def column_mean(x: torch.Tensor, chunk: int = 256) -> torch.Tensor:
     return mean
 
 
-def channel_amax(src: RowSource, tile: int = 1024) -> torch.Tensor:
+def channel_amax(src: RowSource, tile: int | None = None) -> torch.Tensor:
     """Per-(b,h,d) max |x| over S (floored at fp32(1e-4)) as uint32 fp32 bits.
 
-    One workgroup per `tile` rows of a head (the row-tile kernel's largest
-    tile: fewest workgroups and atomics; 64.5 against 72 us at tile 256 for
-    40 x 32768 x 128 bf16 on an MI355X).  The max does not depend on the
-    tiling, so every tile size gives the same bits.
+    One workgroup per `tile` rows of a head: 1024, the row-tile kernel's
+    largest (fewest workgroups and atomics; 64.5 against 72 us at tile 256 for
+    40 x 32768 x 128 bf16 on an MI355X), halved down to 64 while that leaves
+    under two workgroups per CU (2 x 1024 x 64: 10.3 us in two workgroups of
+    1024 rows, 7.3 in 32 of 64).  The max does not depend on the tiling, so
+    every tile size gives the same bits.
     """
     lib = _lib.load()
     b, s, h, d = src.x.shape
+    if tile is None:
+        tile = 1024
+        while tile > 64 and b * h * ((s + tile - 1) // tile) < 512:
+            tile //= 2
     table = torch.empty((b, h, d), dtype=torch.int32, device=src.x.device)
     _lib.check(lib.lbfq_fill_u32(table.data_ptr(), table.numel(), AMAX_FLOOR_BITS,
                                  _lib.stream_handle(src.x.device)), "lbfq_fill_u32")

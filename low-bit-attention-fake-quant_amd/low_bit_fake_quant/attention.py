@@ -191,7 +191,7 @@ def _quant_qk_codes(src: RowSource, cfg: QuantConfig, P: int, *, signs):
     fp8_block -> (B,H,S/block) fp32; mxfp8 -> (B,H,P,D/32) E8M0 bytes."""
     b, s, h, d = src.shape
     dev = src.x.device
-    codes = (torch.zeros if P > s else torch.empty)((b, h, P, d), dtype=torch.uint8, device=dev)
+    codes = torch.empty((b, h, P, d), dtype=torch.uint8, device=dev)  # the kernel zeroes the rows past S
     hs = hadamard_scale(d)
     if cfg.qk_quant == "fp8_block":
         blk = cfg.fp8_block_size
@@ -208,7 +208,7 @@ def _quant_qk_codes(src: RowSource, cfg: QuantConfig, P: int, *, signs):
             raise ValueError(f"D={d} must be divisible by block_d={bd}")
         nb = d // bd
         # padding rows keep E8M0 0 (2^-127): finite, and their codes are zero
-        scale = torch.zeros((b, h, P, nb), dtype=torch.uint8, device=dev)
+        scale = (torch.zeros if P > s else torch.empty)((b, h, P, nb), dtype=torch.uint8, device=dev)
         rowtile(src, R=64, hadamard=cfg.qk_hadamard, signs=signs, had_scale=hs, quant_mode=_lib.Q_MX_QK,
                 codes=codes, codes_layout=_lib.LAYOUT_BHSD, codes_spitch=P, scale=scale,
                 scale_strides=(h * P * nb, nb, P * nb, 1), mx_block=bd, scale_e8m0=True)
@@ -223,7 +223,7 @@ def _quant_v_codes(src: RowSource, cfg: QuantConfig, P: int):
     Returns (codes_t, scale, v_kind, v_block)."""
     b, s, h, d = src.shape
     dev = src.x.device
-    codes = (torch.zeros if P > s else torch.empty)((b, h, d, P), dtype=torch.uint8, device=dev)
+    codes = torch.empty((b, h, d, P), dtype=torch.uint8, device=dev)  # the kernel zeroes the keys past S
     if cfg.v_quant == "fp8_channel":
         table = channel_amax(src)
         scale = torch.empty((b, h, d), dtype=torch.float32, device=dev)
