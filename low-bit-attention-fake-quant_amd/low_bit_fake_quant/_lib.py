@@ -225,4 +225,10 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(device=None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The hipStream_t of torch's current stream on ``device``.  Tensors' devices
+    carry an index, which torch resolves to the raw handle directly (0.2 us;
+    building its Stream object takes 3)."""
+    index = getattr(device, "index", None)
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
