@@ -26,12 +26,12 @@
 // V^T tile from global memory one tile ahead and stage it in a double-buffered
 // LDS area that all its waves read (one barrier per tile).  Scores are
 // computed transposed, S^T = K Q^T: lane (i, g) = (lane % 32, lane / 32)
-// holds query i and, in the MFMA accumulator layout, keys 8 (r / 4) + 4 g +
-// r % 4 (r = 0..15) of each 32-key block.  The PV product O^T = V^T P^T
-// consumes P in that layout: its k-step j of a block contracts the keys of
-// registers r = 8 j .. 8 j + 7, i.e. 16 j + 4 g + {0..3} and 16 j + 8 + 4 g +
-// {0..3} for lane group g; the staged V^T rows hold those eight keys next to
-// each other, so a lane reads its V^T operand as one 16-byte piece.
+// holds query i and, of each 32-key block, the accumulator rows
+// 8 (r / 4) + 4 g + r % 4 (r = 0..15).  K row i of a block is key key_of(i), so
+// that those rows are keys 16 (r / 8) + 8 g + r % 8.  The PV product
+// O^T = V^T P^T consumes P in that layout: its k-step j of a block contracts
+// the keys of registers 8 j .. 8 j + 7, for lane group g the eight consecutive
+// keys 16 j + 8 g + {0..7}, one 16-byte piece of a V^T row.
 #include <cmath>
 
 #include "lbfq_common.h"
@@ -48,7 +48,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
 
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -118,9 +118,7 @@ struct SdpaArgs {
 // double-buffered: the K rows (D bf16 each, pitch KP bytes) and the V^T rows
 // (64 keys each, pitch VP bytes).  The pitches are 16 bytes past a multiple of
 // 128 so that the eight rows one ds_read_b128 phase touches fall on distinct
-// banks.  Within each 16-key group the V^T keys are stored in the order
-// 0-3, 8-11, 4-7, 12-15: lane group g's eight k-elements of a PV k-step are
-// then one contiguous 16-byte read.
+// banks.
 template <int D>
 struct Stage {
   static constexpr int KP = 2 * D + 16;
@@ -156,7 +154,7 @@ __device__ __forceinline__ void stage_load(const uint16_t* kbase, const uint16_t
   }
 }
 
-// registers -> LDS buffer (the key permutation of V^T applied here)
+// registers -> LDS buffer
 template <int D, int NW, bool WITH_V>
 __device__ __forceinline__ void stage_store(uint8_t* buf, int tid, const u32x4 (&kr)[Copy<D, NW>::KCH],
                                             const u32x4 (&vr)[Copy<D, NW>::VCH]) {
@@ -171,13 +169,13 @@ __device__ __forceinline__ void stage_store(uint8_t* buf, int tid, const u32x4 (
 #pragma unroll
     for (int i = 0; i < C::VCH; ++i) {
       const int c = tid + C::T * i, row = c >> 3, kc = c & 7;
-      // keys 16 G + 8 h + [0,4) -> positions 16 G + 4 h + [0,4); + [4,8) -> 16 G + 8 + 4 h + [0,4)
-      uint8_t* rp = buf + Stage<D>::KBYTES + row * Stage<D>::VP + 2 * (16 * (kc >> 1) + 4 * (kc & 1));
-      *reinterpret_cast<u32x2*>(rp) = vr[i].xy;
-      *reinterpret_cast<u32x2*>(rp + 16) = vr[i].zw;
+      *reinterpret_cast<u32x4*>(buf + Stage<D>::KBYTES + row * Stage<D>::VP + 16 * kc) = vr[i];
     }
   }
 }
+
+// Key of K row i of a 32-key block (bits 2 and 3 of i exchanged).
+__device__ __forceinline__ int key_of(int i) { return (i & 0x13) | ((i & 4) << 1) | ((i & 8) >> 1); }
 
 // S^T of the staged tile for the lane's query: two 32-key blocks
 template <int D, int DT>
@@ -185,7 +183,7 @@ __device__ __forceinline__ void scores(const uint8_t* buf, int li, int g, const 
   constexpr int NKS = D / 16;
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb) {
-    const uint8_t* krow = buf + (32 * kb + li) * Stage<D>::KP + 16 * g;
+    const uint8_t* krow = buf + (32 * kb + key_of(li)) * Stage<D>::KP + 16 * g;
     uint4 kop[NKS];
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) kop[ks] = *reinterpret_cast<const uint4*>(krow + 32 * ks);
@@ -197,8 +195,8 @@ __device__ __forceinline__ void scores(const uint8_t* buf, int li, int g, const 
 }
 
 // log2-unit scores of the lane's 32 keys (register r of block kb is key
-// key0 + 32 kb + 8 (r / 4) + 4 g + r % 4); in the tile that holds key S - 1,
-// keys >= S are set to -inf
+// key0 + 32 kb + 16 (r / 8) + 8 g + r % 8); in the tile that holds key S - 1,
+// keys >= S are set to -inf.  brow: the correction of the tile's keys for the lane's query
 template <bool BIAS, int DT>
 __device__ __forceinline__ void to_log2(const v16f (&s)[2], int key0, int g, int S, float sml2, const float* brow,
                                         float (&u)[32]) {
@@ -207,7 +205,7 @@ __device__ __forceinline__ void to_log2(const v16f (&s)[2], int key0, int g, int
     for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
-        const float4 bv = *reinterpret_cast<const float4*>(brow + key0 + 32 * kb + 8 * q4 + 4 * g);
+        const float4 bv = *reinterpret_cast<const float4*>(brow + 32 * kb + 16 * (q4 >> 1) + 8 * g + 4 * (q4 & 1));
         const float bb[4] = {bv.x, bv.y, bv.z, bv.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e)  // the main term rounded to DT first
@@ -228,7 +226,7 @@ __device__ __forceinline__ void to_log2(const v16f (&s)[2], int key0, int g, int
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        if (key0 + 32 * kb + 8 * (r >> 2) + 4 * g + (r & 3) >= S) u[16 * kb + r] = -INFINITY;
+        if (key0 + 32 * kb + 16 * (r >> 3) + 8 * g + (r & 7) >= S) u[16 * kb + r] = -INFINITY;
   }
 }
 
@@ -300,11 +298,45 @@ __device__ __forceinline__ void pv(const uint8_t* buf, int li, int g, const uint
   }
 }
 
-template <int D, bool BIAS, int DT, int NW>
+// Element offset of query qi's output row (its original position).
+template <int D>
+__device__ __forceinline__ size_t out_base(const SdpaArgs& a, int bh, int qi) {
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int orow = a.out_row_map ? a.out_row_map[static_cast<size_t>(bh) * a.S + qi] : qi;
+  return ((static_cast<size_t>(b) * a.S + orow) * a.H + h) * D;
+}
+
+// Four outputs: rounded to the SDPA dtype (the reference's output), then to the caller's dtype.
+template <int DT>
+__device__ __forceinline__ void store_out(const SdpaArgs& a, size_t at, const float (&v)[4]) {
+  float o[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = round_dt<DT>(v[k]);
+  if (a.out_dtype == kF32) {
+    *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.out) + at) = make_float4(o[0], o[1], o[2], o[3]);
+    return;
+  }
+  uint32_t wv[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const uint32_t lo16 = a.out_dtype == kBF16 ? f32_to_bf16_bits(o[2 * k]) : f32_to_f16_bits(o[2 * k]);
+    const uint32_t hi16 = a.out_dtype == kBF16 ? f32_to_bf16_bits(o[2 * k + 1]) : f32_to_f16_bits(o[2 * k + 1]);
+    wv[k] = lo16 | (hi16 << 16);
+  }
+  *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + at) = make_uint2(wv[0], wv[1]);
+}
+
+// BLDS (qm groups of >= 32 queries, so a wave's queries lie in at most two):
+// the correction rows of the tile are staged next to it, one value per lane and
+// row, and read back as LDS broadcasts (8 heads x 32760 x 128: 7.73 -> 7.49 ms).
+// Smaller groups read them from global memory, eight loads a tile whose latency
+// nothing hides.
+template <int D, bool BIAS, bool BLDS, int DT, int NW>
 __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) {
   constexpr int NKS = D / 16, NDB = D / 32;
   using St = Stage<D>;
   __shared__ __align__(16) uint8_t lds[2 * St::BUF];
+  __shared__ __align__(16) float bias_s[BLDS ? 2 : 1][BLDS ? NW : 1][2][BLDS ? 64 : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int li = lane & 31, g = lane >> 5;
@@ -323,12 +355,38 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) qop[ks] = *reinterpret_cast<const uint4*>(qrow + 16 * ks);
   }
-  const float* brow = nullptr;
+  const float* brow = nullptr;         // the lane's correction row
+  const float *b0 = nullptr, *b1 = nullptr;  // the rows of the wave's first and last query
+  int bsel = 0;                        // which of the two is the lane's
   if constexpr (BIAS) {
-    int grp = (qi < S ? qi : S - 1) / a.q_group;
-    grp = grp < a.G ? grp : a.G - 1;
-    brow = a.bias + (static_cast<size_t>(bh) * a.G + grp) * P;
+    auto row_of = [&](int q) {
+      int grp = (q < S ? q : S - 1) / a.q_group;
+      grp = grp < a.G ? grp : a.G - 1;
+      return a.bias + (static_cast<size_t>(bh) * a.G + grp) * P;
+    };
+    brow = row_of(qi);
+    const int q0 = __builtin_amdgcn_readfirstlane(qb * QB + wave * 32);
+    b0 = row_of(q0);
+    b1 = row_of(q0 + 31);
+    bsel = brow == b0 ? 0 : 1;
   }
+  float br0 = 0.0f, br1 = 0.0f;  // the next tile's correction of key `lane`, rows b0 and b1
+  auto bias_load = [&](int key0) {
+    if constexpr (BLDS) {
+      br0 = b0[key0 + lane];
+      br1 = b1[key0 + lane];
+    }
+  };
+  auto bias_store = [&](int slot) {
+    if constexpr (BLDS) {
+      bias_s[slot][wave][0][lane] = br0;
+      bias_s[slot][wave][1][lane] = br1;
+    }
+  };
+  auto bias_tile = [&](int t) -> const float* {
+    if constexpr (BLDS) return bias_s[t & 1][wave][bsel];
+    else return brow + 64 * t;
+  };
   const uint16_t* kbase = a.k + static_cast<size_t>(bh) * P * D;
   const uint16_t* vbase = a.v_t + static_cast<size_t>(bh) * D * P;
   const int nt = (S + 63) / 64;
@@ -345,15 +403,18 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
     // pass 1: the row's max and sum (each lane over its own keys, merged at the end)
     float m = -INFINITY, l = 0.0f;
     stage_load<D, NW, false>(kbase, vbase, P, 0, tid, kr, vr);
+    bias_load(0);
     stage_store<D, NW, false>(lds, tid, kr, vr);
+    bias_store(0);
     __syncthreads();
     for (int t = 0; t < nt; ++t) {
       const uint8_t* buf = lds + (t & 1) * St::BUF;
       v16f s[2];
       scores<D, DT>(buf, li, g, qop, s);
       stage_load<D, NW, false>(kbase, vbase, P, 64 * (t + 1 < nt ? t + 1 : t), tid, kr, vr);
+      bias_load(64 * (t + 1 < nt ? t + 1 : t));
       float u[32];
-      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, brow, u);
+      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, bias_tile(t), u);
       float tmax = u[0];
 #pragma unroll
       for (int j = 1; j < 32; ++j) tmax = fmaxf(tmax, u[j]);
@@ -365,6 +426,7 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
       l = l * __builtin_amdgcn_exp2f(m - ms) + sum;
       m = m_new;
       stage_store<D, NW, false>(lds + ((t + 1) & 1) * St::BUF, tid, kr, vr);  // idle after the last tile
+      bias_store((t + 1) & 1);
       __syncthreads();
     }
     const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
@@ -372,21 +434,25 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
     const float inv = 1.0f / (l * __builtin_amdgcn_exp2f(m - mrow) + lo * __builtin_amdgcn_exp2f(mo - mrow));
     // pass 2: P = dtype(exp2(u - max) / sum), O = P V
     stage_load<D, NW, true>(kbase, vbase, P, 0, tid, kr, vr);
+    bias_load(0);
     stage_store<D, NW, true>(lds, tid, kr, vr);
+    bias_store(0);
     __syncthreads();
     for (int t = 0; t < nt; ++t) {
       const uint8_t* buf = lds + (t & 1) * St::BUF;
       v16f s[2];
       scores<D, DT>(buf, li, g, qop, s);
       stage_load<D, NW, true>(kbase, vbase, P, 64 * (t + 1 < nt ? t + 1 : t), tid, kr, vr);
+      bias_load(64 * (t + 1 < nt ? t + 1 : t));
       float u[32];
-      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, brow, u);
+      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, bias_tile(t), u);
 #pragma unroll
       for (int j = 0; j < 32; ++j) u[j] = __builtin_amdgcn_exp2f(u[j] - mrow) * inv;
       uint32_t w[2][2][4];
       pack<DT>(u, w);
       pv<D, DT>(buf, li, g, w, acc);
       stage_store<D, NW, true>(lds + ((t + 1) & 1) * St::BUF, tid, kr, vr);  // idle after the last tile
+      bias_store((t + 1) & 1);
       __syncthreads();
     }
   } else {
@@ -431,32 +497,203 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
     inv_l = 1.0f / xor32_add(l);
   }
 
-  // epilogue: O rounded to the SDPA dtype (the reference's output), then to the caller's dtype
   if (qi >= S) return;
-  const int b = bh / a.H, h = bh - b * a.H;
-  const int orow = a.out_row_map ? a.out_row_map[static_cast<size_t>(bh) * S + qi] : qi;
-  const size_t obase = ((static_cast<size_t>(b) * S + orow) * a.H + h) * D;
+  const size_t obase = out_base<D>(a, bh, qi);
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) {
-      const int d0 = 32 * db + 8 * r4 + 4 * g;
       float o[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = round_dt<DT>(acc[db][4 * r4 + k] * inv_l);
-      if (a.out_dtype == kF32) {
-        *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.out) + obase + d0) = make_float4(o[0], o[1], o[2], o[3]);
-      } else {
-        uint32_t wv[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const uint32_t lo16 = a.out_dtype == kBF16 ? f32_to_bf16_bits(o[2 * k]) : f32_to_f16_bits(o[2 * k]);
-          const uint32_t hi16 = a.out_dtype == kBF16 ? f32_to_bf16_bits(o[2 * k + 1]) : f32_to_f16_bits(o[2 * k + 1]);
-          wv[k] = lo16 | (hi16 << 16);
-        }
-        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + obase + d0) = make_uint2(wv[0], wv[1]);
-      }
+      for (int k = 0; k < 4; ++k) o[k] = acc[db][4 * r4 + k] * inv_l;
+      store_out<DT>(a, obase + 32 * db + 8 * r4 + 4 * g, o);
     }
+  }
+}
+
+// Small problems: too few 32-query waves to occupy the chip, each a serial
+// chain over all its tiles.  Here a workgroup is 32 queries, and its NW waves
+// take every NW-th 64-key tile each, reading their operands straight from
+// memory (nothing is shared), with the tile's K and V^T loads issued together.
+// The partial results meet in LDS: without a correction each wave's row max,
+// sum and accumulator, rescaled to the common max; with one, the first pass's
+// max and sum meet before the second, which then rounds the same normalised P
+// as sdpa_fwd_kernel, and only accumulators are added.
+template <int D, bool BIAS, int DT, int NW>
+__global__ void __launch_bounds__(NW * 64, 2) sdpa_split_kernel(const SdpaArgs a) {
+  constexpr int NKS = D / 16, NDB = D / 32;
+  __shared__ __align__(16) float acc_s[NW][D / 4][32][4];  // [wave][4 dims][query]
+  __shared__ float m_s[NW][32], l_s[NW][32];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, g = lane >> 5;
+  const int S = a.S, P = a.P;
+  const int nqb = (S + 31) / 32;
+  const int bh = blockIdx.x / nqb, qb = blockIdx.x - bh * nqb;
+  const int qi = qb * 32 + li;  // below the pitch, a multiple of 128
+  uint4 qop[NKS];
+  {
+    const uint16_t* qrow = a.q + (static_cast<size_t>(bh) * P + qi) * D + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) qop[ks] = *reinterpret_cast<const uint4*>(qrow + 16 * ks);
+  }
+  const float* brow = nullptr;
+  if constexpr (BIAS) {
+    int grp = (qi < S ? qi : S - 1) / a.q_group;
+    grp = grp < a.G ? grp : a.G - 1;
+    brow = a.bias + (static_cast<size_t>(bh) * a.G + grp) * P;
+  }
+  const uint16_t* kbase = a.k + static_cast<size_t>(bh) * P * D + key_of(li) * D + 8 * g;
+  const uint16_t* vbase = a.v_t + static_cast<size_t>(bh) * D * P + static_cast<size_t>(li) * P + 8 * g;
+  const int nt = (S + 63) / 64;
+  // V^T operand of k-step j of key block kb, rows 32 db + li
+  auto v_load = [&](int t, uint4 (&vr)[2][2][NDB]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+          vr[kb][j][db] = *reinterpret_cast<const uint4*>(vbase + static_cast<size_t>(32 * db) * P + 64 * t + 32 * kb + 16 * j);
+  };
+  auto tile_scores = [&](int t, v16f (&s)[2]) {
+    uint4 kr[2][NKS];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+        kr[kb][ks] = *reinterpret_cast<const uint4*>(kbase + static_cast<size_t>(64 * t + 32 * kb) * D + 16 * ks);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[kb][r] = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) s[kb] = mfma16<DT>(kr[kb][ks], qop[ks], s[kb]);
+    }
+  };
+  v16f acc[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
+  auto pv_tile = [&](const uint4 (&vr)[2][2][NDB], const uint32_t (&w)[2][2][4]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint4 pb = make_uint4(w[kb][j][0], w[kb][j][1], w[kb][j][2], w[kb][j][3]);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) acc[db] = mfma16<DT>(vr[kb][j][db], pb, acc[db]);
+      }
+  };
+  float m = -INFINITY, l = 0.0f;  // this wave's tiles; with a correction, this lane's keys of them
+  float scale = 1.0f;             // of this wave's accumulator in the sum over waves
+  if constexpr (BIAS) {
+    for (int t = wave; t < nt; t += NW) {
+      v16f s[2];
+      tile_scores(t, s);
+      float u[32];
+      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, brow + 64 * t, u);
+      float tmax = u[0];
+#pragma unroll
+      for (int j = 1; j < 32; ++j) tmax = fmaxf(tmax, u[j]);
+      const float m_new = fmaxf(m, tmax);
+      const float ms = m_new == -INFINITY ? 0.0f : m_new;  // a lane whose keys so far are all masked
+      float sum = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) sum += __builtin_amdgcn_exp2f(u[j] - ms);
+      l = l * __builtin_amdgcn_exp2f(m - ms) + sum;
+      m = m_new;
+    }
+    // the lane pair, then the waves: a wave without tiles, or a pair whose keys
+    // are all masked, has m = -inf and l = 0
+    const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
+    const float mp = fmaxf(m, mo), mps = mp == -INFINITY ? 0.0f : mp;
+    const float lp = l * __builtin_amdgcn_exp2f(m - mps) + lo * __builtin_amdgcn_exp2f(mo - mps);
+    if (g == 0) { m_s[wave][li] = mp; l_s[wave][li] = lp; }
+    __syncthreads();
+    float mrow = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mrow = fmaxf(mrow, m_s[w][li]);  // finite: key 0 is valid
+    float lrow = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) lrow += l_s[w][li] * __builtin_amdgcn_exp2f(m_s[w][li] - mrow);
+    const float inv = 1.0f / lrow;
+    for (int t = wave; t < nt; t += NW) {
+      uint4 vr[2][2][NDB];
+      v_load(t, vr);
+      v16f s[2];
+      tile_scores(t, s);
+      float u[32];
+      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, brow + 64 * t, u);
+#pragma unroll
+      for (int j = 0; j < 32; ++j) u[j] = __builtin_amdgcn_exp2f(u[j] - mrow) * inv;
+      uint32_t w[2][2][4];
+      pack<DT>(u, w);
+      pv_tile(vr, w);
+    }
+  } else {
+    for (int t = wave; t < nt; t += NW) {
+      uint4 vr[2][2][NDB];
+      v_load(t, vr);
+      v16f s[2];
+      tile_scores(t, s);
+      float u[32];
+      to_log2<false, DT>(s, 64 * t, g, S, a.sml2, nullptr, u);
+      float tmax = u[0];
+#pragma unroll
+      for (int j = 1; j < 32; ++j) tmax = fmaxf(tmax, u[j]);
+      const float m_new = fmaxf(m, xor32_max(tmax));  // finite: key 64 t is valid
+      const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 0 on the wave's first tile
+      m = m_new;
+      float sum = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        u[j] = __builtin_amdgcn_exp2f(u[j] - m_new);
+        sum += u[j];
+      }
+      l = l * alpha + sum;
+      if (__any(alpha != 1.0f)) {
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+      }
+      uint32_t whi[2][2][4], wlo[2][2][4];
+      pack_split<DT>(u, whi, wlo);
+      pv_tile(vr, whi);
+      pv_tile(vr, wlo);
+    }
+    const float lp = xor32_add(l);
+    if (g == 0) { m_s[wave][li] = m; l_s[wave][li] = lp; }
+    __syncthreads();
+    float mrow = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mrow = fmaxf(mrow, m_s[w][li]);  // finite: wave 0 holds key 0
+    float lrow = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) lrow += l_s[w][li] * __builtin_amdgcn_exp2f(m_s[w][li] - mrow);
+    scale = __builtin_amdgcn_exp2f(m - mrow) / lrow;  // 0 for a wave without tiles
+  }
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4)
+      *reinterpret_cast<float4*>(&acc_s[wave][8 * db + 2 * r4 + g][li][0]) =
+          make_float4(acc[db][4 * r4] * scale, acc[db][4 * r4 + 1] * scale, acc[db][4 * r4 + 2] * scale,
+                      acc[db][4 * r4 + 3] * scale);
+  __syncthreads();
+  // four dimensions of a query per thread, summed over the waves
+  for (int e = tid; e < 8 * D; e += NW * 64) {
+    const int q = e % 32, d4 = e / 32, qq = qb * 32 + q;
+    if (qq >= S) continue;
+    float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float4 v = *reinterpret_cast<const float4*>(&acc_s[w][d4][q][0]);
+      o[0] += v.x; o[1] += v.y; o[2] += v.z; o[3] += v.w;
+    }
+    store_out<DT>(a, out_base<D>(a, bh, qq) + 4 * d4, o);
   }
 }
 
@@ -588,6 +825,17 @@ extern "C" int lbfq_sdpa_dequant(const lbfq_sdpa_dequant_params* p, lbfq_stream_
   return 0;
 }
 
+// Up to this many 32-query waves (a quarter of the SIMDs) a problem runs
+// sdpa_split_kernel.  Its workgroups each read all of their head's K and V^T,
+// so past that the shared tiles win again.  us, shared tiles -> split:
+//                      waves   plain           with Q smoothing
+//   2 x 1024 x 64         64   20.9 ->  11.8   39.6 ->  18.0
+//   2 x 1024 x 128        64   33.0 ->  20.1   41.2 ->  29.8
+//   1 x 8192 x 128       256  225   -> 128    310   -> 201
+//   4 x 2048 x 128       256   61.1 ->  36.5   82.7 ->  54.6
+//   8 x 2048 x 128       512   62.2 ->  94     78.6 -> 133
+constexpr int64_t kSplitWaves = 256;
+
 extern "C" int lbfq_sdpa_fwd(const lbfq_sdpa_params* p, lbfq_stream_t stream) {
   LBFQ_CHECK_ARG(p, "lbfq_sdpa_fwd: null params");
   LBFQ_CHECK_ARG(p->D == 64 || p->D == 128, "lbfq_sdpa_fwd: D must be 64 or 128");
@@ -620,15 +868,32 @@ extern "C" int lbfq_sdpa_fwd(const lbfq_sdpa_params* p, lbfq_stream_t stream) {
   const dim3 grid(static_cast<unsigned>(w8 ? nwg8 : p->B * p->H * (p->s_pitch / 128))), block(w8 ? 512 : 256);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool bias = p->qk_bias != nullptr, bf = p->sdpa_dtype == kBF16;
-#define LBFQ_SD(DD, BI, DT)                                                             \
-  do {                                                                                  \
-    if (w8) hipLaunchKernelGGL((sdpa_fwd_kernel<DD, BI, DT, 8>), grid, block, 0, st, a); \
-    else hipLaunchKernelGGL((sdpa_fwd_kernel<DD, BI, DT, 4>), grid, block, 0, st, a);    \
+  // few 32-query waves: eight waves share one's keys (kSplitWaves below)
+  const int64_t nw32 = p->B * p->H * ((p->S + 31) / 32);
+  if (nw32 <= kSplitWaves && p->S > 64) {
+    const dim3 gs(static_cast<unsigned>(nw32)), bs(512);
+#define LBFQ_SP(DD, BI)                                                                            \
+  do {                                                                                             \
+    if (bf) hipLaunchKernelGGL((sdpa_split_kernel<DD, BI, kBF16, 8>), gs, bs, 0, st, a);           \
+    else hipLaunchKernelGGL((sdpa_split_kernel<DD, BI, kF16, 8>), gs, bs, 0, st, a);               \
   } while (0)
-#define LBFQ_SD_DT(DD, BI) \
-  if (bf) LBFQ_SD(DD, BI, kBF16); else LBFQ_SD(DD, BI, kF16)
-#define LBFQ_SD_BI(DD) \
-  if (bias) { LBFQ_SD_DT(DD, true); } else { LBFQ_SD_DT(DD, false); }
+    if (p->D == 128) { if (bias) LBFQ_SP(128, true); else LBFQ_SP(128, false); }
+    else { if (bias) LBFQ_SP(64, true); else LBFQ_SP(64, false); }
+#undef LBFQ_SP
+    LBFQ_LAUNCH_CHECK("lbfq_sdpa_fwd (split)");
+    return 0;
+  }
+  const bool blds = bias && p->q_group >= 32;
+#define LBFQ_SD(DD, BI, BL, DT)                                                             \
+  do {                                                                                      \
+    if (w8) hipLaunchKernelGGL((sdpa_fwd_kernel<DD, BI, BL, DT, 8>), grid, block, 0, st, a); \
+    else hipLaunchKernelGGL((sdpa_fwd_kernel<DD, BI, BL, DT, 4>), grid, block, 0, st, a);    \
+  } while (0)
+#define LBFQ_SD_DT(DD, BI, BL) \
+  if (bf) LBFQ_SD(DD, BI, BL, kBF16); else LBFQ_SD(DD, BI, BL, kF16)
+#define LBFQ_SD_BI(DD)                                                                                     \
+  if (blds) { LBFQ_SD_DT(DD, true, true); } else if (bias) { LBFQ_SD_DT(DD, true, false); } \
+  else { LBFQ_SD_DT(DD, false, false); }
   if (p->D == 128) { LBFQ_SD_BI(128) } else { LBFQ_SD_BI(64) }
 #undef LBFQ_SD_BI
 #undef LBFQ_SD_DT
