@@ -188,12 +188,27 @@ struct AssignLds {
   uint4 part[2][D / 16][MB][64];   // hi / lo operands, as the lanes read them
   float cent[32 * MB * P];
   float cn[32 * MB];
-  float a0[32 * MB];               // -cn / 2, the MFMA accumulators' start; far below any other for rows >= K
+  float a0[32 * MB];               // -cn / 2, the MFMA accumulators' start; far below any other for rows that never win
+  float c2max;                     // >= max_j |c_j|^2; infinity if a centroid is not finite
+  uint64_t twins;                  // centroids that a later row repeats
 };
+
+// The largest of the lanes' values, which are not negative; infinity if one is not finite.
+__device__ __forceinline__ float wave_top(float v) {
+  v = v < INFINITY ? v : INFINITY;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
+  return v;
+}
 
 // The centroids of slice bh into LDS: fp32 rows, hi / lo MFMA operands and the
 // norms (the specification's chain).  Rows K .. 32 MB - 1 are zero with norm
-// +inf, so they never win.
+// +inf, so they never win; nor does a row that repeats an earlier one bit by
+// bit, as its scores are the earlier row's and the first minimum wins.  Repeats
+// are what a padded sequence brings (its pad tokens are one row, and an initial
+// centroid is every S / K-th token): left in, they tie in every round, and each
+// pad token takes the full settle: a round over 8 x 512 x 128 with 140 tokens of
+// padding took 50 us with 32 clusters and 97 with 64, against 11 and 14 here.
 template <int D, int MB>
 __device__ __forceinline__ void assign_fill(AssignLds<D, MB>& lds, const float* cent, int K) {
   using L = AssignLds<D, MB>;
@@ -211,20 +226,46 @@ __device__ __forceinline__ void assign_fill(AssignLds<D, MB>& lds, const float* 
     lds.part[1][c8 / 2][j / 32][j % 32 + 32 * (c8 & 1)] = __builtin_bit_cast(uint4, lo);
   }
   __syncthreads();
-  if (threadIdx.x < 32 * MB) {
-    const float4* c = reinterpret_cast<const float4*>(lds.cent + threadIdx.x * L::P);
+  if (threadIdx.x < 64) {  // one wave
+    const int j = threadIdx.x < 32 * MB ? threadIdx.x : 0;
+    const uint4* row = reinterpret_cast<const uint4*>(lds.cent + j * L::P);
     float acc = 0.0f;
 #pragma unroll 8
     for (int i = 0; i < D / 4; ++i) {
-      const float4 v = c[i];
+      const float4 v = __builtin_bit_cast(float4, row[i]);
       acc = fmaf(v.x, v.x, acc);
       acc = fmaf(v.y, v.y, acc);
       acc = fmaf(v.z, v.z, acc);
       acc = fmaf(v.w, v.w, acc);
     }
     const bool real = static_cast<int>(threadIdx.x) < K;
-    lds.cn[threadIdx.x] = real ? acc : INFINITY;
-    lds.a0[threadIdx.x] = real ? -0.5f * acc : -1e38f;
+    // the first row of this norm, then whether all of it is the same
+    const int bits = __float_as_int(acc);
+    int first = j;
+    for (int jo = K - 1; jo >= 0; --jo) first = __builtin_amdgcn_readlane(bits, jo) == bits && jo < first ? jo : first;
+    bool repeat = real && first < j;
+    if (__any(repeat)) {
+      const uint4* row0 = reinterpret_cast<const uint4*>(lds.cent + first * L::P);
+      uint32_t diff = 0u;
+#pragma unroll 8
+      for (int i = 0; i < D / 4; ++i) {
+        const uint4 v = row[i], v0 = row0[i];
+        diff |= (v.x ^ v0.x) | (v.y ^ v0.y) | (v.z ^ v0.z) | (v.w ^ v0.w);
+      }
+      repeat = repeat && diff == 0u;
+    }
+    uint64_t twins = 0ull;
+    for (uint64_t m = __ballot(repeat); m; m &= m - 1)
+      twins |= 1ull << __builtin_amdgcn_readlane(first, __builtin_ctzll(m));
+    const float c2max = wave_top(real ? acc : 0.0f);
+    if (threadIdx.x < 32 * MB) {
+      lds.cn[j] = real && !repeat ? acc : INFINITY;
+      lds.a0[j] = real && !repeat ? -0.5f * acc : -1e38f;
+    }
+    if (threadIdx.x == 0) {
+      lds.c2max = c2max;
+      lds.twins = twins;
+    }
   }
   __syncthreads();
 }
@@ -237,14 +278,6 @@ __device__ __forceinline__ uint32_t from_pair(uint32_t v, int g) {
 }
 __device__ __forceinline__ float from_pair(float v, int g) {
   return __uint_as_float(from_pair(__float_as_uint(v), g));
-}
-
-// The largest of the lanes' values, which are not negative; infinity if one is not finite.
-__device__ __forceinline__ float wave_top(float v) {
-  v = v < INFINITY ? v : INFINITY;
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
 }
 
 // The specification for one token (its row at element x0) per PER lanes: lane
@@ -364,6 +397,7 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
   const bool filter = tr.ul && prev_changed;
   int64_t cur = -1;
   float c2max = 0.0f, cmax = 0.0f;  // >= max_j |c_j|^2; the slice's cum_max of this round
+  uint64_t twins = 0ull;
   for (int64_t w = w0; w < w1;) {
     const int64_t bh = w / nslab, s_in = w - bh * nslab;
     int64_t ns = w1 - w < kSeg ? w1 - w : kSeg;
@@ -374,7 +408,8 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
       if (cur >= 0) __syncthreads();  // every wave is done with the previous slice's centroids
       assign_fill<D, MB>(lds, cent + bh * K * D, K);
       cur = bh;
-      c2max = wave_top(lane < K ? lds.cn[lane] : 0.0f);
+      c2max = lds.c2max;
+      twins = lds.twins;
       if (tr.ul) {
         if (static_cast<int>(threadIdx.x) < K) cum_s[threadIdx.x] = tr.cum[bh * K + threadIdx.x];
         cmax = 0.0f;
@@ -569,7 +604,7 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
         // the stored norms) below the gap and that of |x|^2 below 2^-15 of it
         const float e = gap + 0x1p-15f * xx;
         float2 st = make_float2(INFINITY, 0.0f);  // never holds
-        if (settled) {
+        if (settled && !(twins >> bj & 1)) {  // a repeat of the label's centroid is as near as that, and may part from it
           st.x = __builtin_amdgcn_sqrtf(fmaxf(xx - 2.0f * top, 0.0f) + e) * (1.0f + kOut) - cum_s[bj];
           st.y = __builtin_amdgcn_sqrtf(fmaxf(xx - 2.0f * second - e, 0.0f)) * (1.0f - kOut) + cmax;
         }
@@ -600,9 +635,12 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
 // fp64 per-cluster column sums of one kChunk-token chunk.  The chunk's tokens
 // are first sorted by label in LDS, stably (ballot ranks within a wave, waves
 // and rounds in token order), so a cluster's tokens keep their order.  Then
-// the D / 8 lanes of group g -- 8 columns each, one 16-byte load per bf16 row --
-// add the runs of clusters j = g, g + NG, ... in that order: the token-order
-// fp64 sums of the specification, with 8 rows in flight per lane.
+// wave g -- D / 64 columns a lane -- adds the runs of clusters j = g, g + 8, ...
+// in that order: the token-order fp64 sums of the specification, with kPf rows
+// in flight.  A whole wave to a row, because clusters are uneven: the pad
+// tokens of a short sequence are one cluster.  With 8 columns a lane and 16 lanes
+// to a cluster, 512 tokens with 240 of them padding waited for one chain of 30
+// batches of 8 rows, 45 us a round against 19 (first round 70 against 31).
 //
 // The first round also finds out whether the chunk's sums are exact: values
 // are multiples of the smallest nonzero one's last bit, and a sum of up to
@@ -614,22 +652,54 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
 // unless more than a quarter of the chunk moved.
 //
 // Bound by the row reads and the LDS sort ahead of them: at 40 x 32768 x 128
-// bf16 with 32 clusters the first round (the ranges included) takes 125 us, the
-// later ones 67, 31, 18, then 14 as fewer tokens move (every round 132 us with
-// one column and a 2-byte load per lane and no moves).
+// bf16 with 32 clusters the first round (the ranges included) takes 97 us, the
+// later ones 60, 25, 18, then 15 as fewer tokens move; with 64 clusters 119, 83,
+// 52, then 45 to 35 (16 lanes to a cluster: 125, 67, 31, 18, 14, and every
+// round 132 us with one column and a 2-byte load per lane and no moves).
 constexpr int kUpdThreads = 512;
 constexpr int kMaxMoved = kChunk / 4;
+
+// a lane's share of a row: D / 64 consecutive columns of dtype DT
+template <int D, int DT>
+struct Cols {
+  static constexpr int C = D / 64;
+  using Mag = typename Raw8<DT>::Mag;
+  using Word = std::conditional_t<DT == kF32, std::conditional_t<C == 2, uint2, uint32_t>,
+                                  std::conditional_t<C == 2, uint32_t, uint16_t>>;
+  Word w;
+  __device__ __forceinline__ void load(const uint8_t* row, int lane) { w = reinterpret_cast<const Word*>(row)[lane]; }
+  __device__ __forceinline__ void to_f32(float (&v)[C]) const {
+    if constexpr (DT == kF32) {
+      if constexpr (C == 2) { v[0] = __uint_as_float(w.x); v[1] = __uint_as_float(w.y); }
+      else v[0] = __uint_as_float(w);
+    } else {
+#pragma unroll
+      for (int k = 0; k < C; ++k) {
+        const uint16_t e = static_cast<uint16_t>(w >> (16 * k));
+        v[k] = DT == kBF16 ? bf16_bits_to_f32(e) : f16_bits_to_f32(e);
+      }
+    }
+  }
+  __device__ __forceinline__ void range(Mag& big, Mag& small) const {
+    if constexpr (DT == kF32 && C == 2) {
+      Raw8<DT>::range_word(w.x, big, small);
+      Raw8<DT>::range_word(w.y, big, small);
+    } else {
+      Raw8<DT>::range_word(w, big, small);  // a 16-bit word's upper half, zero, counts as none
+    }
+  }
+};
 
 template <int D, int DT>
 __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const void* x, int64_t S, int64_t H, int K,
                                                                         const int32_t* labels, double* partial,
                                                                         int32_t* counts, const int32_t* changed,
                                                                         const Track tr, int first) {
-  constexpr int LPG = D / 8;             // lanes per cluster group
-  constexpr int NG = kUpdThreads / LPG;  // cluster groups
+  using Share = Cols<D, DT>;
+  constexpr int C = Share::C;
   constexpr int NW = kUpdThreads / 64;
-  constexpr int kPf = DT == kF32 ? 4 : 8;  // rows in flight per lane
-  constexpr int kGone = 1 << 16;           // move entry: the row left the cluster
+  constexpr int kPf = DT == kF32 ? 16 : 32;  // rows in flight per wave
+  constexpr int kGone = 1 << 16;             // move entry: the row left the cluster
   __shared__ int lab_s[kChunk];  // label; moved tokens: + (previous label + 1) << 8
   __shared__ int ord_s[kChunk];  // rows in cluster order, or the moves in cluster order
   __shared__ int start_s[kMaxKAssign + 1];
@@ -641,13 +711,52 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
   const int64_t bh = blockIdx.x / nchunk, c = blockIdx.x % nchunk;
   if (changed[bh] == 0) return;  // converged slice (uniform per workgroup)
   const int64_t b = bh / H, h = bh % H;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t t0 = c * kChunk;
   const int n = static_cast<int>(t0 + kChunk < S ? kChunk : S - t0);
-  const int g = tid / LPG, col = 8 * (tid % LPG);
-  double* const out = partial + (bh * nchunk + c) * K * D + col;
+  double* const out = partial + (bh * nchunk + c) * K * D + C * lane;
   int32_t* const cnt_out = counts + (bh * nchunk + c) * K;
-  const int64_t xrow0 = (b * S + t0) * H + h;
+  const int64_t pitch = H * D * (DT == kF32 ? 4 : 2);
+  const uint8_t* const row0 = static_cast<const uint8_t*>(x) + (b * S + t0) * pitch + h * D * (DT == kF32 ? 4 : 2);
+  typename Share::Mag big = 0, small = ~big;
+  // acc += the rows of entries p0 .. p1 - 1 in order (MOVES: minus those that
+  // left; RANGES: their magnitudes as well).  Past p1 a group of 8 repeats the
+  // last row as +0, which changes no sum (one that starts at +0 is never -0).
+  auto add_run = [&](int p0, int p1, double (&acc)[C], auto MOVES, auto RANGES) {
+    for (; p0 < p1; p0 += kPf) {
+      const int mine = ord_s[p0 + lane < p1 ? p0 + lane : p1 - 1];
+      Share raw[kPf];
+#pragma unroll
+      for (int i = 0; i < kPf; i += 8) {
+        if (p0 + i < p1) {
+#pragma unroll
+          for (int k = i; k < i + 8; ++k) {
+            const int r = __builtin_amdgcn_readlane(mine, k);
+            raw[k].load(row0 + (MOVES ? r & (kGone - 1) : r) * pitch, lane);
+          }
+        }
+      }
+      asm volatile("" ::: "memory");  // all of them issued before the first is waited for
+#pragma unroll
+      for (int i = 0; i < kPf; i += 8) {
+        if (p0 + i < p1) {
+#pragma unroll
+          for (int k = i; k < i + 8; ++k) {
+            float v[C];
+            raw[k].to_f32(v);
+            const uint32_t keep = p0 + k < p1 ? ~0u : 0u;
+            const uint32_t neg = MOVES ? static_cast<uint32_t>(__builtin_amdgcn_readlane(mine, k) & kGone) << 15 & keep : 0u;
+#pragma unroll
+            for (int e = 0; e < C; ++e)
+              acc[e] += static_cast<double>(__uint_as_float((__float_as_uint(v[e]) & keep) ^ neg));
+            if (RANGES) raw[k].range(big, small);
+          }
+        }
+      }
+    }
+  };
+  using std::false_type;
+  using std::true_type;
   const bool by_moves = tr.ul && !first && tr.exact[bh * nchunk + c] != 0;  // if few enough moved
   for (int i = tid; i < K; i += kUpdThreads) { start_s[i + 1] = 0; running[i] = 0; net_s[i] = 0; }
   for (int i = tid; i < NW * K; i += kUpdThreads) wcnt[i / K][i % K] = 0;
@@ -711,38 +820,15 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
       cnt_out[tid] += net_s[tid];
       tr.touched[bh * K + tid] = 1;
     }
-    for (int j = g; j < K; j += NG) {
-      const int p1 = start_s[j + 1];
-      int p0 = start_s[j];
+    for (int j = wave; j < K; j += NW) {
+      const int p0 = start_s[j], p1 = start_s[j + 1];
       if (p0 == p1) continue;
-      double2* o = reinterpret_cast<double2*>(out + j * D);
-      double acc[8];
+      double acc[C];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double2 v = o[k];
-        acc[2 * k] = v.x;
-        acc[2 * k + 1] = v.y;
-      }
-      for (; p0 < p1; p0 += kPf) {
-        Raw8<DT> raw[kPf];
+      for (int k = 0; k < C; ++k) acc[k] = out[j * D + k];
+      add_run(p0, p1, acc, true_type{}, false_type{});
 #pragma unroll
-        for (int i = 0; i < kPf; ++i) {
-          const int r = ord_s[p0 + i < p1 ? p0 + i : p1 - 1] & (kGone - 1);
-          raw[i].load(x, (xrow0 + static_cast<int64_t>(r) * H) * D + col);
-        }
-#pragma unroll
-        for (int i = 0; i < kPf; ++i) {
-          if (p0 + i < p1) {
-            float v[8];
-            raw[i].to_f32(v);
-            const float sg = ord_s[p0 + i] & kGone ? -1.0f : 1.0f;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(sg * v[k]);
-          }
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
+      for (int k = 0; k < C; ++k) out[j * D + k] = acc[k];
     }
     return;
   }
@@ -778,34 +864,13 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     cnt_out[tid] = start_s[tid + 1] - start_s[tid];
     if (tr.ul) tr.touched[bh * K + tid] = 1;
   }
-  // column sums over the sorted runs of this group's clusters
-  typename Raw8<DT>::Mag big = 0, small = ~big;
-  for (int j = g; j < K; j += NG) {
-    const int p1 = start_s[j + 1];
-    double acc[8];
+  // column sums over the sorted runs of this wave's clusters
+  for (int j = wave; j < K; j += NW) {
+    double acc[C] = {};
+    if (first) add_run(start_s[j], start_s[j + 1], acc, false_type{}, true_type{});
+    else add_run(start_s[j], start_s[j + 1], acc, false_type{}, false_type{});
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc[k] = 0.0;
-    for (int p0 = start_s[j]; p0 < p1; p0 += kPf) {
-      Raw8<DT> raw[kPf];
-#pragma unroll
-      for (int i = 0; i < kPf; ++i) {
-        const int pos = p0 + i < p1 ? p0 + i : p1 - 1;
-        raw[i].load(x, (xrow0 + static_cast<int64_t>(ord_s[pos]) * H) * D + col);
-      }
-#pragma unroll
-      for (int i = 0; i < kPf; ++i) {
-        if (p0 + i < p1) {
-          float v[8];
-          raw[i].to_f32(v);
-#pragma unroll
-          for (int k = 0; k < 8; ++k) acc[k] += static_cast<double>(v[k]);
-          if (first) raw[i].range(big, small);
-        }
-      }
-    }
-    double2* o = reinterpret_cast<double2*>(out + j * D);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) o[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
+    for (int k = 0; k < C; ++k) out[j * D + k] = acc[k];
   }
   if (tr.ul && first) {
     atomicMax(&range_s[0], Raw8<DT>::widest(big, true));

@@ -78,6 +78,21 @@ def test_rounds_that_reuse_the_last(gpu, kind, dtype):
         _check(x.to(dtype), gpu, k, iters=iters, seed=iters)
 
 
+@pytest.mark.parametrize("pad", ["zeros", "last_row"])
+@pytest.mark.parametrize("s,k,dtype", [(272, 32, torch.bfloat16), (372, 64, torch.bfloat16), (300, 40, torch.float32)])
+def test_repeated_centroids(gpu, s, k, dtype, pad):
+    """A padded sequence starts with many centroids that are one and the same
+    row; the first of them moves off with its cluster's other tokens, and the
+    pad tokens go to the next repeat."""
+    g = torch.Generator().manual_seed(s)
+    x = torch.randn(2, 512, 3, 64, generator=g)
+    x[:, :s // 2] *= 0.1   # tokens that share the pad rows' cluster at first
+    x[:, s - 1] *= 0.1
+    x[:, s:] = 0.0 if pad == "zeros" else x[:, s - 1:s]
+    for iters in (1, 2, 3, 10):
+        _check(x.to(dtype), gpu, k, iters=iters, seed=iters)
+
+
 def test_noalloc_without_room_for_the_carried_state(gpu):
     """A problem that fits the built-in scratch only without the state carried
     between rounds still runs there, with the same labels."""
