@@ -79,6 +79,13 @@ typedef struct {
 
 int lbfq_rowtile(const lbfq_rowtile_params* p, lbfq_stream_t stream);
 
+/* Quantises p0 and, unless it is null, p1 (quant modes FP8_BLOCK and MX_QK), as
+ * two lbfq_rowtile calls would, and sets fill[0 .. fill_n) to fill_value (null
+ * and 0 for none): one launch where both problems have the same dtype, mode,
+ * Hadamard flag and kind of sub_mode (none or some). */
+int lbfq_rowtile_pair(const lbfq_rowtile_params* p0, const lbfq_rowtile_params* p1, uint32_t* fill, int64_t fill_n,
+                      uint32_t fill_value, lbfq_stream_t stream);
+
 /* Sequential fp64 column sums over `chunk`-row chunks (optionally gathered):
  * mode 0 -> partial (B, nchunk, H, D) fp64; mode 1 -> mean fp32 per chunk.
  * Replaces the reductions of preprocess.py:10-36 (smooth_k, mode 0 +

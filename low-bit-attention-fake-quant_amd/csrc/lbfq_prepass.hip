@@ -174,7 +174,7 @@ __device__ __forceinline__ void zero_padding(const RowTileArgs& a, int64_t bh, i
 }
 
 template <int DT, int QM, bool SUB, bool HAD>
-__global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a) {
+__device__ __forceinline__ void rowtile_body(const RowTileArgs& a, uint32_t block) {
   constexpr bool TILE_RED = QM == LBFQ_Q_FP8_BLOCK || QM == LBFQ_Q_MX_V || QM == LBFQ_Q_CHANNEL_AMAX;
   constexpr bool RESIDENT_MODE = QM == LBFQ_Q_FP8_BLOCK || QM == LBFQ_Q_MX_V;
   constexpr int ES = DT == kF32 ? 4 : 2;  // input element bytes
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a)
   // below 2^31
   const uint32_t ntile = a.ntile;
   const uint32_t H32 = static_cast<uint32_t>(a.H);
-  uint32_t t = blockIdx.x;
+  uint32_t t = block;
   const int64_t h = t % H32;
   t /= H32;
   const int64_t tile = t % ntile;
@@ -526,6 +526,34 @@ __global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a)
   }
 }
 
+template <int DT, int QM, bool SUB, bool HAD>
+__global__ void __launch_bounds__(kTileWaves * 64) rowtile_kernel(RowTileArgs a) {
+  rowtile_body<DT, QM, SUB, HAD>(a, blockIdx.x);
+}
+
+// Two problems of one kind in one launch, workgroups [0, n0) and [n0, ...), and
+// a table filled beside them: a small call is bound by its launches (2 x 1024 x
+// 64: Q, K and the table of V's maxima are 4 to 5 us each, most of it the
+// launch).  The register counts are rowtile_kernel's, so a large call loses
+// nothing (12 x 32760 x 128, all codes and scales: 199 -> 198 us).
+struct RowTilePair {
+  RowTileArgs a[2];
+  uint32_t n0;
+  uint32_t* fill;
+  int64_t fill_n;
+  uint32_t fill_value;
+};
+
+template <int DT, int QM, bool SUB, bool HAD>
+__global__ void __launch_bounds__(kTileWaves * 64) rowtile_pair_kernel(RowTilePair p) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * (kTileWaves * 64) + threadIdx.x; i < p.fill_n;
+       i += static_cast<int64_t>(gridDim.x) * (kTileWaves * 64))
+    p.fill[i] = p.fill_value;
+  const bool second = blockIdx.x >= p.n0;
+  const RowTileArgs a = second ? p.a[1] : p.a[0];
+  rowtile_body<DT, QM, SUB, HAD>(a, second ? blockIdx.x - p.n0 : blockIdx.x);
+}
+
 // Sequential fp64 column sums of `chunk` rows (optionally gathered).
 // mode 0: write fp64 partial sums (B, nchunk, H, D);
 // mode 1: write fp32 means fp32(sum / rows_in_chunk) (B, nchunk, H, D).
@@ -691,7 +719,17 @@ void launch_rowtile(int qm, bool sub, bool had, dim3 grid, dim3 block, size_t sh
 
 }  // namespace
 
-extern "C" int lbfq_rowtile(const lbfq_rowtile_params* p, lbfq_stream_t stream) {
+namespace {
+
+// A checked problem: its kernel arguments and launch.
+struct RowTileLaunch {
+  RowTileArgs a;
+  unsigned grid;
+  size_t shmem;
+  bool sub, had;
+};
+
+int rowtile_prepare(const lbfq_rowtile_params* p, RowTileLaunch* out) {
   LBFQ_CHECK_ARG(p && p->x, "lbfq_rowtile: null input");
   LBFQ_CHECK_ARG(p->D == 64 || p->D == 128, "lbfq_rowtile: D must be 64 or 128; got %lld", (long long)p->D);
   LBFQ_CHECK_ARG(p->x_dtype >= 0 && p->x_dtype <= 2, "lbfq_rowtile: bad dtype %d", p->x_dtype);
@@ -720,7 +758,8 @@ extern "C" int lbfq_rowtile(const lbfq_rowtile_params* p, lbfq_stream_t stream) 
   LBFQ_CHECK_ARG(p->codes_layout != LBFQ_LAYOUT_BHDS || p->codes_spitch % 4 == 0,
                  "lbfq_rowtile: transposed codes pitch must be a multiple of 4");
   LBFQ_CHECK_ARG(p->codes_layout == LBFQ_LAYOUT_NHD || p->codes_spitch >= p->S, "lbfq_rowtile: bad codes pitch");
-  RowTileArgs a;
+  RowTileArgs& a = out->a;
+  a = RowTileArgs{};
   a.x = p->x; a.x_dtype = p->x_dtype; a.B = p->B; a.S = p->S; a.H = p->H; a.D = p->D; a.R = p->R;
   a.gather = p->gather; a.sub_mode = p->sub_mode; a.sub = p->sub; a.sub_block = p->sub_block;
   a.smoothed = p->smoothed; a.hadamard = p->hadamard; a.signs = p->signs; a.had_scale = p->had_scale;
@@ -737,14 +776,74 @@ extern "C" int lbfq_rowtile(const lbfq_rowtile_params* p, lbfq_stream_t stream) 
   const int64_t nblocks = ntiles;  // one workgroup per tile
   LBFQ_CHECK_ARG(nblocks < (1ll << 31), "lbfq_rowtile: grid too large");
   LBFQ_CHECK_ARG(p->R % (512 / p->D) == 0, "lbfq_rowtile: R must be a multiple of %lld", (long long)(512 / p->D));
-  size_t shmem = p->codes_layout == LBFQ_LAYOUT_BHDS ? static_cast<size_t>(kStageRows * (p->D + 4)) : 0;
-  const dim3 grid(static_cast<unsigned>(nblocks)), block(kTileWaves * 64);
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool sub = p->sub_mode != LBFQ_SUB_NONE, had = p->hadamard != 0;
-  if (p->x_dtype == kBF16) launch_rowtile<kBF16>(qm, sub, had, grid, block, shmem, st, a);
-  else if (p->x_dtype == kF16) launch_rowtile<kF16>(qm, sub, had, grid, block, shmem, st, a);
-  else launch_rowtile<kF32>(qm, sub, had, grid, block, shmem, st, a);
+  out->shmem = p->codes_layout == LBFQ_LAYOUT_BHDS ? static_cast<size_t>(kStageRows * (p->D + 4)) : 0;
+  out->grid = static_cast<unsigned>(nblocks);
+  out->sub = p->sub_mode != LBFQ_SUB_NONE;
+  out->had = p->hadamard != 0;
+  return 0;
+}
+
+void rowtile_launch(const RowTileLaunch& l, hipStream_t st) {
+  const dim3 grid(l.grid), block(kTileWaves * 64);
+  const int dt = l.a.x_dtype, qm = l.a.quant_mode;
+  if (dt == kBF16) launch_rowtile<kBF16>(qm, l.sub, l.had, grid, block, l.shmem, st, l.a);
+  else if (dt == kF16) launch_rowtile<kF16>(qm, l.sub, l.had, grid, block, l.shmem, st, l.a);
+  else launch_rowtile<kF32>(qm, l.sub, l.had, grid, block, l.shmem, st, l.a);
+}
+
+template <int DT, int QM>
+void launch_pair_qm(const RowTilePair& p, bool sub, bool had, unsigned grid, size_t shmem, hipStream_t st) {
+  const dim3 g(grid), block(kTileWaves * 64);
+  if (sub && had) hipLaunchKernelGGL((rowtile_pair_kernel<DT, QM, true, true>), g, block, shmem, st, p);
+  else if (sub) hipLaunchKernelGGL((rowtile_pair_kernel<DT, QM, true, false>), g, block, shmem, st, p);
+  else if (had) hipLaunchKernelGGL((rowtile_pair_kernel<DT, QM, false, true>), g, block, shmem, st, p);
+  else hipLaunchKernelGGL((rowtile_pair_kernel<DT, QM, false, false>), g, block, shmem, st, p);
+}
+
+template <int DT>
+void launch_pair(const RowTilePair& p, int qm, bool sub, bool had, unsigned grid, size_t shmem, hipStream_t st) {
+  if (qm == LBFQ_Q_MX_QK) launch_pair_qm<DT, LBFQ_Q_MX_QK>(p, sub, had, grid, shmem, st);
+  else launch_pair_qm<DT, LBFQ_Q_FP8_BLOCK>(p, sub, had, grid, shmem, st);
+}
+
+}  // namespace
+
+extern "C" int lbfq_rowtile(const lbfq_rowtile_params* p, lbfq_stream_t stream) {
+  RowTileLaunch l;
+  const int rc = rowtile_prepare(p, &l);
+  if (rc) return rc;
+  rowtile_launch(l, static_cast<hipStream_t>(stream));
   LBFQ_LAUNCH_CHECK("lbfq_rowtile");
+  return 0;
+}
+
+extern "C" int lbfq_rowtile_pair(const lbfq_rowtile_params* p0, const lbfq_rowtile_params* p1, uint32_t* fill,
+                                 int64_t fill_n, uint32_t fill_value, lbfq_stream_t stream) {
+  RowTileLaunch l[2];
+  int rc = rowtile_prepare(p0, &l[0]);
+  if (!rc && p1) rc = rowtile_prepare(p1, &l[1]);
+  if (rc) return rc;
+  LBFQ_CHECK_ARG(fill_n >= 0 && (fill || fill_n == 0), "lbfq_rowtile_pair: bad fill table");
+  const int qm = p0->quant_mode;
+  LBFQ_CHECK_ARG(qm == LBFQ_Q_FP8_BLOCK || qm == LBFQ_Q_MX_QK, "lbfq_rowtile_pair: quant modes FP8_BLOCK and MX_QK only");
+  // one launch where both run the same kernel; else the second follows on its own
+  const bool one = p1 && p1->quant_mode == qm && p1->x_dtype == p0->x_dtype && l[1].sub == l[0].sub &&
+                   l[1].had == l[0].had && l[1].shmem == l[0].shmem &&
+                   static_cast<int64_t>(l[0].grid) + l[1].grid < (int64_t{1} << 31);
+  RowTilePair p{};
+  p.a[0] = l[0].a;
+  p.a[1] = one ? l[1].a : l[0].a;
+  p.n0 = l[0].grid;
+  p.fill = fill;
+  p.fill_n = fill_n;
+  p.fill_value = fill_value;
+  const unsigned grid = l[0].grid + (one ? l[1].grid : 0u);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (p0->x_dtype == kBF16) launch_pair<kBF16>(p, qm, l[0].sub, l[0].had, grid, l[0].shmem, st);
+  else if (p0->x_dtype == kF16) launch_pair<kF16>(p, qm, l[0].sub, l[0].had, grid, l[0].shmem, st);
+  else launch_pair<kF32>(p, qm, l[0].sub, l[0].had, grid, l[0].shmem, st);
+  if (p1 && !one) rowtile_launch(l[1], st);
+  LBFQ_LAUNCH_CHECK("lbfq_rowtile_pair");
   return 0;
 }
 

@@ -703,9 +703,8 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_split_kernel(const SdpaArgs a
 // 8 elements per thread.  qk_mx 0: scale (BH, S / blk) fp32 per blk rows;
 // 1: scale (BH, P, D / blk) E8M0 per blk columns.
 template <int DT>
-__global__ void qk_dequant_kernel(const uint8_t* codes, int qk_mx, const void* scale, int blk, int64_t BH, int S,
-                                  int P, int D, uint16_t* out) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void qk_dequant(int64_t t, const uint8_t* codes, int qk_mx, const void* scale, int blk,
+                                           int64_t BH, int S, int P, int D, uint16_t* out) {
   const int per_row = D / 8;
   if (t >= BH * P * per_row) return;
   const int c8 = static_cast<int>(t % per_row);
@@ -733,9 +732,9 @@ __global__ void qk_dequant_kernel(const uint8_t* codes, int qk_mx, const void* s
 // keys >= S zero.  8 keys per thread.  v_kind 0: scale (BH, D) fp32; 1: (BH, S / vb)
 // fp32; 2: (BH, S / vb, D) E8M0.  alpha: (BH, S / vsb, D) fp32 or null.
 template <int DT>
-__global__ void v_dequant_t_kernel(const uint8_t* codes_t, int v_kind, const void* scale, int vb, const float* alpha,
-                                   int vsb, int64_t BH, int S, int P, int D, uint16_t* out) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void v_dequant_t(int64_t t, const uint8_t* codes_t, int v_kind, const void* scale, int vb,
+                                            const float* alpha, int vsb, int64_t BH, int S, int P, int D,
+                                            uint16_t* out) {
   const int per_row = P / 8;
   if (t >= BH * D * per_row) return;
   const int k0 = 8 * static_cast<int>(t % per_row);
@@ -776,6 +775,21 @@ __global__ void v_dequant_t_kernel(const uint8_t* codes_t, int v_kind, const voi
   reinterpret_cast<uint4*>(out)[t] = o;
 }
 
+// Q, K and V^T (grid y: 0, 1, 2; all three have B H P D elements) in one
+// launch: a small call is bound by its launches (2 x 1024 x 64: a whole call takes
+// 72 us with three here and three more for the Q and K codes and the table of V
+// maxima, 60 with one of each kind).
+template <int DT>
+__global__ void sdpa_dequant_kernel(const lbfq_sdpa_dequant_params p, int64_t BH, int S, int P, int D) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (blockIdx.y == 2)
+    v_dequant_t<DT>(t, p.v_codes_t, p.v_kind, p.v_scale, p.v_block, p.v_alpha, p.v_smooth_block, BH, S, P, D,
+                    static_cast<uint16_t*>(p.v_t_out));
+  else
+    qk_dequant<DT>(t, blockIdx.y ? p.k_codes : p.q_codes, p.qk_mx, blockIdx.y ? p.k_scale : p.q_scale, p.qk_block, BH,
+                   S, P, D, static_cast<uint16_t*>(blockIdx.y ? p.k_out : p.q_out));
+}
+
 }  // namespace
 
 extern "C" int lbfq_sdpa_dequant(const lbfq_sdpa_dequant_params* p, lbfq_stream_t stream) {
@@ -800,27 +814,11 @@ extern "C" int lbfq_sdpa_dequant(const lbfq_sdpa_dequant_params* p, lbfq_stream_
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t BH = p->B * p->H;
   const int S = static_cast<int>(p->S), P = static_cast<int>(p->s_pitch), D = static_cast<int>(p->D);
-  const dim3 gqk(static_cast<unsigned>((BH * P * (D / 8) + 255) / 256)), gv(static_cast<unsigned>((BH * D * (P / 8) + 255) / 256));
-  const dim3 block(256);
-  const bool bf = p->sdpa_dtype == kBF16;
-  const void* codes[2] = {p->q_codes, p->k_codes};
-  const void* scales[2] = {p->q_scale, p->k_scale};
-  void* outs[2] = {p->q_out, p->k_out};
-  for (int i = 0; i < 2; ++i) {
-    const uint8_t* c = static_cast<const uint8_t*>(codes[i]);
-    uint16_t* o = static_cast<uint16_t*>(outs[i]);
-    if (bf)
-      hipLaunchKernelGGL(qk_dequant_kernel<kBF16>, gqk, block, 0, st, c, p->qk_mx, scales[i], p->qk_block, BH, S, P, D, o);
-    else
-      hipLaunchKernelGGL(qk_dequant_kernel<kF16>, gqk, block, 0, st, c, p->qk_mx, scales[i], p->qk_block, BH, S, P, D, o);
-  }
-  uint16_t* vo = static_cast<uint16_t*>(p->v_t_out);
-  if (bf)
-    hipLaunchKernelGGL(v_dequant_t_kernel<kBF16>, gv, block, 0, st, p->v_codes_t, p->v_kind, p->v_scale, p->v_block,
-                       p->v_alpha, p->v_smooth_block, BH, S, P, D, vo);
+  const dim3 grid(static_cast<unsigned>((BH * P * (D / 8) + 255) / 256), 3), block(256);
+  if (p->sdpa_dtype == kBF16)
+    hipLaunchKernelGGL(sdpa_dequant_kernel<kBF16>, grid, block, 0, st, *p, BH, S, P, D);
   else
-    hipLaunchKernelGGL(v_dequant_t_kernel<kF16>, gv, block, 0, st, p->v_codes_t, p->v_kind, p->v_scale, p->v_block,
-                       p->v_alpha, p->v_smooth_block, BH, S, P, D, vo);
+    hipLaunchKernelGGL(sdpa_dequant_kernel<kF16>, grid, block, 0, st, *p, BH, S, P, D);
   LBFQ_LAUNCH_CHECK("lbfq_sdpa_dequant");
   return 0;
 }

@@ -150,6 +150,8 @@ class SdpaParams(ctypes.Structure):
 _SIGS = {
     "lbfq_last_error": (ctypes.c_char_p, []),
     "lbfq_rowtile": (_i32, [ctypes.POINTER(RowTileParams), _vp]),
+    "lbfq_rowtile_pair": (_i32, [ctypes.POINTER(RowTileParams), ctypes.POINTER(RowTileParams), _vp, _i64,
+                                 ctypes.c_uint32, _vp]),
     "lbfq_colsum": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _i32, _vp, _i32, _vp, _vp, _vp]),
     "lbfq_colsum_finalize": (_i32, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp]),
     "lbfq_fill_u32": (_i32, [_vp, _i64, ctypes.c_uint32, _vp]),

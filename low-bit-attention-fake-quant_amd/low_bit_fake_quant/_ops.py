@@ -39,12 +39,11 @@ class RowSource:
         return self.x.shape
 
 
-def rowtile(src: RowSource, *, R: int, smoothed: torch.Tensor | None = None, smoothed_stage: int = 0,
-            signs: torch.Tensor | None = None, hadamard: bool = False, had_scale: float = 1.0,
-            quant_mode: int = _lib.Q_NONE, codes: torch.Tensor | None = None, codes_layout: int = _lib.LAYOUT_NHD,
-            codes_spitch: int = 0, scale: torch.Tensor | None = None, scale_strides=(0, 0, 0, 0),
-            amax_table: torch.Tensor | None = None, mx_block: int = 32, scale_e8m0: bool = False) -> None:
-    lib = _lib.load()
+def rowtile_params(src: RowSource, *, R: int, smoothed: torch.Tensor | None = None, smoothed_stage: int = 0,
+                   signs: torch.Tensor | None = None, hadamard: bool = False, had_scale: float = 1.0,
+                   quant_mode: int = _lib.Q_NONE, codes: torch.Tensor | None = None, codes_layout: int = _lib.LAYOUT_NHD,
+                   codes_spitch: int = 0, scale: torch.Tensor | None = None, scale_strides=(0, 0, 0, 0),
+                   amax_table: torch.Tensor | None = None, mx_block: int = 32, scale_e8m0: bool = False) -> _lib.RowTileParams:
     x = src.x
     b, s, h, d = x.shape
     p = _lib.RowTileParams()
@@ -63,7 +62,19 @@ def rowtile(src: RowSource, *, R: int, smoothed: torch.Tensor | None = None, smo
     p.mx_block = int(mx_block)
     p.smoothed_stage = int(smoothed_stage)
     p.scale_e8m0 = 1 if scale_e8m0 else 0
-    _lib.check(lib.lbfq_rowtile(p, _lib.stream_handle(x.device)), "lbfq_rowtile")
+    return p
+
+
+def rowtile(src: RowSource, **kw) -> None:
+    _lib.check(_lib.load().lbfq_rowtile(rowtile_params(src, **kw), _lib.stream_handle(src.x.device)), "lbfq_rowtile")
+
+
+def rowtile_pair(p0, p1, device, amax_table: torch.Tensor | None = None) -> None:
+    """Quantise one or two (p1 may be None) Q / K problems; amax_table, if
+    given, starts at the channel maxima's floor (for channel_amax)."""
+    n = 0 if amax_table is None else amax_table.numel()
+    _lib.check(_lib.load().lbfq_rowtile_pair(p0, p1, _lib.ptr(amax_table), n, AMAX_FLOOR_BITS,
+                                             _lib.stream_handle(device)), "lbfq_rowtile_pair")
 
 
 def colsum_mean(x: torch.Tensor, chunk: int, gather: torch.Tensor | None = None) -> torch.Tensor:
@@ -91,8 +102,9 @@ def column_mean(x: torch.Tensor, chunk: int = 256) -> torch.Tensor:
     return mean
 
 
-def channel_amax(src: RowSource, tile: int | None = None) -> torch.Tensor:
-    """Per-(b,h,d) max |x| over S (floored at fp32(1e-4)) as uint32 fp32 bits.
+def channel_amax(src: RowSource, tile: int | None = None, table: torch.Tensor | None = None) -> torch.Tensor:
+    """Per-(b,h,d) max |x| over S (floored at fp32(1e-4)) as uint32 fp32 bits,
+    into ``table`` if given (which holds the floor already).
 
     One workgroup per `tile` rows of a head: 1024, the row-tile kernel's
     largest (fewest workgroups and atomics; 64.5 against 72 us at tile 256 for
@@ -101,15 +113,15 @@ def channel_amax(src: RowSource, tile: int | None = None) -> torch.Tensor:
     1024 rows, 7.3 in 32 of 64).  The max does not depend on the tiling, so
     every tile size gives the same bits.
     """
-    lib = _lib.load()
     b, s, h, d = src.x.shape
     if tile is None:
         tile = 1024
         while tile > 64 and b * h * ((s + tile - 1) // tile) < 512:
             tile //= 2
-    table = torch.empty((b, h, d), dtype=torch.int32, device=src.x.device)
-    _lib.check(lib.lbfq_fill_u32(table.data_ptr(), table.numel(), AMAX_FLOOR_BITS,
-                                 _lib.stream_handle(src.x.device)), "lbfq_fill_u32")
+    if table is None:
+        table = torch.empty((b, h, d), dtype=torch.int32, device=src.x.device)
+        _lib.check(_lib.load().lbfq_fill_u32(table.data_ptr(), table.numel(), AMAX_FLOOR_BITS,
+                                             _lib.stream_handle(src.x.device)), "lbfq_fill_u32")
     rowtile(src, R=tile, quant_mode=_lib.Q_CHANNEL_AMAX, amax_table=table)
     return table
 

@@ -33,7 +33,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._ops import RowSource, channel_amax, colsum_mean, column_mean, hadamard_scale, qmk, round_up, rowtile
+from ._ops import RowSource, channel_amax, colsum_mean, column_mean, hadamard_scale, qmk, round_up, rowtile, rowtile_pair, rowtile_params
 from .attention_kernel import launch_attention, v_tile_colsum, validate_kernel_config
 from .config import QuantConfig
 from .hadamard import apply_qk_hadamard, qk_signs_device
@@ -186,9 +186,10 @@ def _kmeans_result(src_tensor, km) -> Optional[KMeansReorderResult]:
 # ---------------------------------------------------------------------------
 
 
-def _quant_qk_codes(src: RowSource, cfg: QuantConfig, P: int, *, signs):
-    """Quantise one of Q/K into head-major codes (B,H,P,D) and the kernel's scales:
-    fp8_block -> (B,H,S/block) fp32; mxfp8 -> (B,H,P,D/32) E8M0 bytes."""
+def _qk_codes(src: RowSource, cfg: QuantConfig, P: int, *, signs):
+    """One of Q/K as head-major codes (B,H,P,D) with the kernel's scales:
+    fp8_block -> (B,H,S/block) fp32; mxfp8 -> (B,H,P,D/32) E8M0 bytes.  Returns
+    (codes, scale, the quantiser's parameters); rowtile_pair fills both."""
     b, s, h, d = src.shape
     dev = src.x.device
     codes = torch.empty((b, h, P, d), dtype=torch.uint8, device=dev)  # the kernel zeroes the rows past S
@@ -199,7 +200,7 @@ def _quant_qk_codes(src: RowSource, cfg: QuantConfig, P: int, *, signs):
             raise ValueError(f"S={s} must be divisible by block_s={blk}")
         nb = s // blk
         scale = torch.empty((b, h, nb), dtype=torch.float32, device=dev)
-        rowtile(src, R=blk, hadamard=cfg.qk_hadamard, signs=signs, had_scale=hs, quant_mode=_lib.Q_FP8_BLOCK,
+        p = rowtile_params(src, R=blk, hadamard=cfg.qk_hadamard, signs=signs, had_scale=hs, quant_mode=_lib.Q_FP8_BLOCK,
                 codes=codes, codes_layout=_lib.LAYOUT_BHSD, codes_spitch=P, scale=scale,
                 scale_strides=(h * nb, 1, nb, 0))
     elif cfg.qk_quant == "mxfp8":
@@ -209,23 +210,29 @@ def _quant_qk_codes(src: RowSource, cfg: QuantConfig, P: int, *, signs):
         nb = d // bd
         # padding rows keep E8M0 0 (2^-127): finite, and their codes are zero
         scale = (torch.zeros if P > s else torch.empty)((b, h, P, nb), dtype=torch.uint8, device=dev)
-        rowtile(src, R=64, hadamard=cfg.qk_hadamard, signs=signs, had_scale=hs, quant_mode=_lib.Q_MX_QK,
+        p = rowtile_params(src, R=64, hadamard=cfg.qk_hadamard, signs=signs, had_scale=hs, quant_mode=_lib.Q_MX_QK,
                 codes=codes, codes_layout=_lib.LAYOUT_BHSD, codes_spitch=P, scale=scale,
                 scale_strides=(h * P * nb, nb, P * nb, 1), mx_block=bd, scale_e8m0=True)
     else:
         raise ValueError(f"unsupported qk_quant: {cfg.qk_quant!r}")
-    return codes, scale
+    return codes, scale, p
 
 
-def _quant_v_codes(src: RowSource, cfg: QuantConfig, P: int):
+def _amax_table(src: RowSource, cfg: QuantConfig) -> Optional[torch.Tensor]:
+    """The channel maxima's table of a V that is quantised per channel."""
+    b, _, h, d = src.shape
+    return torch.empty((b, h, d), dtype=torch.int32, device=src.x.device) if cfg.v_quant == "fp8_channel" else None
+
+
+def _quant_v_codes(src: RowSource, cfg: QuantConfig, P: int, table: Optional[torch.Tensor]):
     """Quantise V into transposed codes (B,H,D,P) and the kernel's scales:
     channel (B,H,D) fp32, fp8_block (B,H,S/vb) fp32, mxfp8 (B,H,S/vb,D) E8M0.
-    Returns (codes_t, scale, v_kind, v_block)."""
+    ``table``: _amax_table's, filled.  Returns (codes_t, scale, v_kind, v_block)."""
     b, s, h, d = src.shape
     dev = src.x.device
     codes = torch.empty((b, h, d, P), dtype=torch.uint8, device=dev)  # the kernel zeroes the keys past S
     if cfg.v_quant == "fp8_channel":
-        table = channel_amax(src)
+        channel_amax(src, table=table)
         scale = torch.empty((b, h, d), dtype=torch.float32, device=dev)
         rowtile(src, R=64, quant_mode=_lib.Q_CHANNEL, codes=codes, codes_layout=_lib.LAYOUT_BHDS, codes_spitch=P,
                 scale=scale, scale_strides=(scale.stride(0), 0, scale.stride(1), scale.stride(2)), amax_table=table)
@@ -292,16 +299,19 @@ def quantize_operands(prep: _Prep, cfg: QuantConfig, sm_scale: float) -> Quantiz
             raise ValueError("rowmax_mode='qm_k' requires smoothing='full' so qm exists")
     elif cfg.rowmax_mode != "online":
         raise ValueError(f"unsupported rowmax_mode: {cfg.rowmax_mode!r}")
-    q_codes, q_scale = _quant_qk_codes(prep.q, cfg, P, signs=signs)
+    q_codes, q_scale, pq = _qk_codes(prep.q, cfg, P, signs=signs)
     # with the qm correction, K_s is quantised inside the qm.K_s pass when it can be
     fuse_k = has_qm and _k_quant_fusable(prep.k, cfg, P, prep.qm.shape[1])
     if fuse_k:
         blk = cfg.fp8_block_size
         k_codes = (torch.zeros if P > s else torch.empty)((b, h, P, d), dtype=torch.uint8, device=prep.k.x.device)
         k_scale = torch.empty((b, h, s // blk), dtype=torch.float32, device=prep.k.x.device)
+        pk = None
     else:
-        k_codes, k_scale = _quant_qk_codes(prep.k, cfg, P, signs=signs)
-    v_codes, v_scale, v_kind, v_block = _quant_v_codes(prep.v, cfg, P)
+        k_codes, k_scale, pk = _qk_codes(prep.k, cfg, P, signs=signs)
+    amax = _amax_table(prep.v, cfg)
+    rowtile_pair(pq, pk, prep.q.x.device, amax)
+    v_codes, v_scale, v_kind, v_block = _quant_v_codes(prep.v, cfg, P, amax)
     bias = rowmax = None
     if has_qm:
         # scores are handled in log2 units by the kernel
@@ -427,9 +437,11 @@ def sdpa_operands(prep: _Prep, cfg: QuantConfig, sm_scale: float, sdpa_dtype: to
     signs = None
     if cfg.qk_hadamard and cfg.qk_hadamard_random_sign:
         signs = qk_signs_device(h, d, cfg.qk_hadamard_seed, dev)
-    q_codes, q_scale = _quant_qk_codes(prep.q, cfg, P, signs=signs)
-    k_codes, k_scale = _quant_qk_codes(prep.k, cfg, P, signs=signs)
-    v_codes, v_scale, v_kind, v_block = _quant_v_codes(prep.v, cfg, P)
+    q_codes, q_scale, pq = _qk_codes(prep.q, cfg, P, signs=signs)
+    k_codes, k_scale, pk = _qk_codes(prep.k, cfg, P, signs=signs)
+    amax = _amax_table(prep.v, cfg)
+    rowtile_pair(pq, pk, dev, amax)
+    v_codes, v_scale, v_kind, v_block = _quant_v_codes(prep.v, cfg, P, amax)
     v_alpha = None
     if prep.v_alpha is not None:
         if s % cfg.v_smooth_block_size != 0:
