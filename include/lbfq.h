@@ -110,7 +110,9 @@ int lbfq_dequant(const uint8_t* codes, const float* scale, int64_t B, int64_t S,
  * x: NHD tensor; per (b, h) slice cluster S tokens of dimension D into K
  * clusters with `iters` Lloyd rounds (deterministic init from `seed`).
  * Workspace: centroids (B*H, K, D) fp32, partial (B*H, ceil(S/1024), K, D)
- * fp64, counts (B*H, ceil(S/1024), K) int32.  Outputs labels / order /
+ * fp64, counts (B*H, ceil(S/1024), K) int32, and the state that a round leaves
+ * for the next: distance bounds (B*H, S, 2) fp32 and summed labels (B*H, S)
+ * bytes, with a few words per centroid and chunk.  Outputs labels / order /
  * inverse as (B*H, S) int32. */
 int64_t lbfq_kmeans_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int K);
 int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int K, int iters,
@@ -122,7 +124,9 @@ int lbfq_kmeans(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64
  * serving loops, harnesses that forbid hipMalloc.  Same kernels and results
  * as lbfq_kmeans; the workspace is a built-in device array of
  * lbfq_kmeans_noalloc_max_workspace_bytes() (64 MiB) per GPU, held until the
- * process ends.  Returns -1 when lbfq_kmeans_workspace_bytes() exceeds it.
+ * process ends.  A problem whose workspace exceeds it runs without the state
+ * carried between rounds, more slowly; returns -1 when the rest exceeds it
+ * too (K * D * (8 * ceil(S/1024) + 4) bytes per slice and a little more).
  * Calls that overlap on one GPU share that array and race. */
 int64_t lbfq_kmeans_noalloc_max_workspace_bytes(void);
 int lbfq_kmeans_noalloc(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int K, int iters,

@@ -656,8 +656,14 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
 // later ones 60, 25, 18, then 15 as fewer tokens move; with 64 clusters 119, 83,
 // 52, then 45 to 35 (16 lanes to a cluster: 125, 67, 31, 18, 14, and every
 // round 132 us with one column and a 2-byte load per lane and no moves).
+//
+// Where one chunk is the slice, `cent` is not null and the centroids follow at
+// once: with a pass of its own ten rounds over 2 x 512 x 128 take 366 us, 295 so.
 constexpr int kUpdThreads = 512;
 constexpr int kMaxMoved = kChunk / 4;
+
+// the length of a centroid's step, from above; s: the sum of its squares
+__device__ __forceinline__ float step_length(float s) { return 1.001f * sqrtf(s + 0x1p-120f); }
 
 // a lane's share of a row: D / 64 consecutive columns of dtype DT
 template <int D, int DT>
@@ -691,10 +697,11 @@ struct Cols {
 };
 
 template <int D, int DT>
-__global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const void* x, int64_t S, int64_t H, int K,
+__global__ void __launch_bounds__(kUpdThreads, 8) km_update_partial_kernel(const void* x, int64_t S, int64_t H, int K,
                                                                         const int32_t* labels, double* partial,
                                                                         int32_t* counts, const int32_t* changed,
-                                                                        const Track tr, int first) {
+                                                                        const Track tr, int first, float* cent,
+                                                                        int32_t* clear_next) {
   using Share = Cols<D, DT>;
   constexpr int C = Share::C;
   constexpr int NW = kUpdThreads / 64;
@@ -709,6 +716,7 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
   __shared__ uint32_t range_s[2];  // largest magnitude; smallest nonzero one, minus 1 (bits)
   const int64_t nchunk = (S + kChunk - 1) / kChunk;
   const int64_t bh = blockIdx.x / nchunk, c = blockIdx.x % nchunk;
+  if (clear_next && threadIdx.x == 0) clear_next[bh] = 0;
   if (changed[bh] == 0) return;  // converged slice (uniform per workgroup)
   const int64_t b = bh / H, h = bh % H;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -780,7 +788,32 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     }
     if (by_moves) moved += __syncthreads_count(mv);
   }
-  if (by_moves && moved == 0) return;
+  // a slice of one chunk: the sums are the slice's, so this is its centroid pass too
+  auto centroid = [&](int j, const double (&acc)[C], int cnt) {
+    float* cp = cent + (bh * K + j) * D + C * lane;
+    float now[C], s = 0.0f;
+#pragma unroll
+    for (int e = 0; e < C; ++e) {
+      const float old = cp[e];
+      now[e] = cnt > 0 ? static_cast<float>(acc[e] / static_cast<double>(cnt)) : old;
+      s += (now[e] - old) * (now[e] - old);
+    }
+#pragma unroll
+    for (int e = 0; e < C; ++e) cp[e] = now[e];
+    if (tr.ul) {
+#pragma unroll
+      for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m, 64);
+      if (lane == 0) {
+        const float step = step_length(s);
+        tr.delta[bh * K + j] = step;
+        tr.cum[bh * K + j] += step;
+      }
+    }
+  };
+  if (by_moves && moved == 0) {
+    if (cent && tid < K) tr.delta[bh * K + tid] = 0.0f;
+    return;
+  }
   const bool moves = by_moves && moved <= kMaxMoved;
   __syncthreads();
   // histogram and starts of the clusters' runs
@@ -815,20 +848,28 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
         ord_s[start_s[old] + atomicAdd(&running[old], 1)] = i | kGone;
       }
     }
-    __syncthreads();
-    if (tid < K && start_s[tid + 1] > start_s[tid]) {
-      cnt_out[tid] += net_s[tid];
-      tr.touched[bh * K + tid] = 1;
+    if (tid < K) {
+      const int cnt = cnt_out[tid] + net_s[tid];
+      net_s[tid] = cnt;
+      if (start_s[tid + 1] > start_s[tid]) {
+        cnt_out[tid] = cnt;
+        tr.touched[bh * K + tid] = 1;
+      }
     }
+    __syncthreads();
     for (int j = wave; j < K; j += NW) {
       const int p0 = start_s[j], p1 = start_s[j + 1];
-      if (p0 == p1) continue;
+      if (p0 == p1) {
+        if (cent && lane == 0) tr.delta[bh * K + j] = 0.0f;
+        continue;
+      }
       double acc[C];
 #pragma unroll
       for (int k = 0; k < C; ++k) acc[k] = out[j * D + k];
       add_run(p0, p1, acc, true_type{}, false_type{});
 #pragma unroll
       for (int k = 0; k < C; ++k) out[j * D + k] = acc[k];
+      if (cent) centroid(j, acc, net_s[j]);
     }
     return;
   }
@@ -871,6 +912,7 @@ __global__ void __launch_bounds__(kUpdThreads) km_update_partial_kernel(const vo
     else add_run(start_s[j], start_s[j + 1], acc, false_type{}, false_type{});
 #pragma unroll
     for (int k = 0; k < C; ++k) out[j * D + k] = acc[k];
+    if (cent) centroid(j, acc, start_s[j + 1] - start_s[j]);
   }
   if (tr.ul && first) {
     atomicMax(&range_s[0], Raw8<DT>::widest(big, true));
@@ -936,7 +978,7 @@ __global__ void __launch_bounds__(D) km_finalize_kernel(const double* partial, c
     __syncthreads();  // also: every thread has read touched
     if (d == 0) {
       if (D == 128) s += red[1];
-      const float step = 1.001f * sqrtf(s + 0x1p-120f);
+      const float step = step_length(s);
       tr.delta[bh * K + j] = step;
       tr.cum[bh * K + j] += step;
       tr.touched[bh * K + j] = 0;
@@ -1113,8 +1155,9 @@ int kmeans_run(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_
   for (int it = 0; it < rounds; ++it) {
     const dim3 ga(nasg), gu(static_cast<unsigned>(BH * nchunk));
     // round it writes flag slot it % 2, read by its update and finalize and by
-    // round it + 1's assignment; finalize clears slot (it + 1) % 2 first
+    // round it + 1's assignment; the centroid pass clears slot (it + 1) % 2 first
     int32_t* cur = w.changed + (it & 1) * BH;
+    int32_t* clear = w.changed + ((it + 1) & 1) * BH;
     const int32_t* prev = it == 0 ? nullptr : w.changed + ((it - 1) & 1) * BH;
 #define LBFQ_KM(DD, DT)                                                                                             \
   if (K <= 32)                                                                                                      \
@@ -1125,7 +1168,8 @@ int kmeans_run(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_
                        prev, cur, w.track, it);                                                                     \
   if (it + 1 < rounds)                                                                                              \
     hipLaunchKernelGGL((km_update_partial_kernel<DD, DT>), gu, dim3(kUpdThreads), 0, st, x, S, H, K, labels,        \
-                       w.partial, w.counts, cur, w.track, it == 0);
+                       w.partial, w.counts, cur, w.track, it == 0, nchunk == 1 ? w.cent : nullptr,                \
+                       nchunk == 1 ? clear : nullptr);
     if (D == 128) {
       if (dtype == kBF16) { LBFQ_KM(128, kBF16) } else if (dtype == kF16) { LBFQ_KM(128, kF16) } else { LBFQ_KM(128, kF32) }
     } else {
@@ -1134,7 +1178,7 @@ int kmeans_run(const void* x, int dtype, int64_t B, int64_t S, int64_t H, int64_
 #undef LBFQ_KM
     LBFQ_LAUNCH_CHECK("km_assign / km_update_partial");
     if (it + 1 == rounds) break;  // the last update does not change the labels
-    int32_t* clear = w.changed + ((it + 1) & 1) * BH;
+    if (nchunk == 1) continue;  // done by the update
     const dim3 gf(static_cast<unsigned>(BH * K));
     if (D == 128)
       hipLaunchKernelGGL(km_finalize_kernel<128>, gf, dim3(128), 0, st, w.partial, w.counts, nchunk, K, w.cent, cur,

@@ -93,12 +93,14 @@ def test_repeated_centroids(gpu, s, k, dtype, pad):
         _check(x.to(dtype), gpu, k, iters=iters, seed=iters)
 
 
-def test_noalloc_without_room_for_the_carried_state(gpu):
+@pytest.mark.parametrize("s,h", [(60 << 16, 2), (1024, 8192)])
+def test_noalloc_without_room_for_the_carried_state(gpu, s, h):
     """A problem that fits the built-in scratch only without the state carried
-    between rounds still runs there, with the same labels."""
+    between rounds (long slices, and many of one chunk) still runs there, with
+    the same labels."""
     from low_bit_fake_quant import _lib as L
     lib = L.load()
-    b, s, h, d, k = 1, 60 << 16, 2, 64, 8
+    b, d, k = 1, 64, 8
     need = int(lib.lbfq_kmeans_workspace_bytes(b, s, h, d, k))
     assert need > int(lib.lbfq_kmeans_noalloc_max_workspace_bytes())
     x = torch.randn(b, s, h, d, device=gpu, dtype=torch.bfloat16)
