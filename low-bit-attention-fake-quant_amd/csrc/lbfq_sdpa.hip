@@ -197,7 +197,7 @@ __device__ __forceinline__ void scores(const uint8_t* buf, int li, int g, const 
 // log2-unit scores of the lane's 32 keys (register r of block kb is key
 // key0 + 32 kb + 16 (r / 8) + 8 g + r % 8); in the tile that holds key S - 1,
 // keys >= S are set to -inf.  brow: the correction of the tile's keys for the lane's query
-template <bool BIAS, int DT>
+template <bool BIAS, int DT, bool FENCE = true, bool MASK = true>
 __device__ __forceinline__ void to_log2(const v16f (&s)[2], int key0, int g, int S, float sml2, const float* brow,
                                         float (&u)[32]) {
   if constexpr (BIAS) {
@@ -213,7 +213,7 @@ __device__ __forceinline__ void to_log2(const v16f (&s)[2], int key0, int g, int
       }
       // the second block's correction loads stay behind the first block's use
       // (all eight in flight at once took the kernel past 256 VGPRs)
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
     }
   } else {
 #pragma unroll
@@ -221,7 +221,7 @@ __device__ __forceinline__ void to_log2(const v16f (&s)[2], int key0, int g, int
 #pragma unroll
       for (int r = 0; r < 16; ++r) u[16 * kb + r] = s[kb][r] * sml2;
   }
-  if (key0 + 64 > S) {
+  if (MASK && key0 + 64 > S) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -406,15 +406,22 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
     bias_load(0);
     stage_store<D, NW, false>(lds, tid, kr, vr);
     bias_store(0);
+    stage_load<D, NW, false>(kbase, vbase, P, nt > 1 ? 64 : 0, tid, kr, vr);
+    stage_store<D, NW, false>(lds + St::BUF, tid, kr, vr);
     __syncthreads();
-    for (int t = 0; t < nt; ++t) {
-      const uint8_t* buf = lds + (t & 1) * St::BUF;
-      v16f s[2];
-      scores<D, DT>(buf, li, g, qop, s);
-      stage_load<D, NW, false>(kbase, vbase, P, 64 * (t + 1 < nt ? t + 1 : t), tid, kr, vr);
+    v16f s0[2], s1[2];
+    scores<D, DT>(lds, li, g, qop, s0);
+    __syncthreads();
+    // one tile: its softmax sums beside the products of the next, whose K is
+    // staged already (past the last tile they are not used), an MFMA to every 12
+    // VALU instructions: 8 heads x 32760 x 128 7.49 -> 7.20 ms.  The same in pass 2
+    // gained nothing more, and with four waves it spills.
+    auto step = [&](int t, const v16f (&s)[2], v16f (&sn)[2], auto MASK) {
+      stage_load<D, NW, false>(kbase, vbase, P, 64 * (t + 2 < nt ? t + 2 : nt - 1), tid, kr, vr);
       bias_load(64 * (t + 1 < nt ? t + 1 : t));
+      scores<D, DT>(lds + ((t + 1) & 1) * St::BUF, li, g, qop, sn);
       float u[32];
-      to_log2<true, DT>(s, 64 * t, g, S, a.sml2, bias_tile(t), u);
+      to_log2<true, DT, false, MASK>(s, 64 * t, g, S, a.sml2, bias_tile(t), u);
       float tmax = u[0];
 #pragma unroll
       for (int j = 1; j < 32; ++j) tmax = fmaxf(tmax, u[j]);
@@ -425,10 +432,25 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_fwd_kernel(const SdpaArgs a) 
       for (int j = 0; j < 32; ++j) sum += __builtin_amdgcn_exp2f(u[j] - ms);
       l = l * __builtin_amdgcn_exp2f(m - ms) + sum;
       m = m_new;
-      stage_store<D, NW, false>(lds + ((t + 1) & 1) * St::BUF, tid, kr, vr);  // idle after the last tile
+      if constexpr (!MASK) {
+#pragma unroll
+        for (int i = 0; i < 2 * NKS; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
+        }
+      }
+      stage_store<D, NW, false>(lds + (t & 1) * St::BUF, tid, kr, vr);
       bias_store((t + 1) & 1);
       __syncthreads();
+    };
+    int t = 0;
+    for (; t + 2 < nt; t += 2) {
+      step(t, s0, s1, std::false_type{});
+      step(t + 1, s1, s0, std::false_type{});
     }
+    step(t, s0, s1, std::true_type{});
+    if (t + 1 < nt) step(t + 1, s1, s0, std::true_type{});
     const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
     const float mrow = fmaxf(m, mo);  // finite: key 0 is valid
     const float inv = 1.0f / (l * __builtin_amdgcn_exp2f(m - mrow) + lo * __builtin_amdgcn_exp2f(mo - mrow));
