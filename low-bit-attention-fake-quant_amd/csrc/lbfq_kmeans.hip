@@ -182,14 +182,19 @@ constexpr int kAsgThreads = 64 * kAsgWaves;
 constexpr int kSlab = 32 * kAsgWaves;  // tokens per slab: one 32-token step of each wave
 constexpr int kSeg = 8;                // slabs of a segment at most
 
+// Below every a_j where c2max is finite: |c_j|^2 < 1e38 then, and a finite gap
+// bounds x.c by X C < 2^64, so a_j > -0.51e38.  From 1e38 on c2max is infinite,
+// no gap is finite and every token takes the full settle.
+constexpr float kNeverWins = -1e38f;
+
 template <int D, int MB>
 struct AssignLds {
   static constexpr int P = D + 4;  // row pitch of the fp32 centroids: float4 reads of 16 rows hit distinct banks
   uint4 part[2][D / 16][MB][64];   // hi / lo operands, as the lanes read them
   float cent[32 * MB * P];
   float cn[32 * MB];
-  float a0[32 * MB];               // -cn / 2, the MFMA accumulators' start; far below any other for rows that never win
-  float c2max;                     // >= max_j |c_j|^2; infinity if a centroid is not finite
+  float a0[32 * MB];               // -cn / 2, the MFMA accumulators' start; kNeverWins for rows that never win
+  float c2max;                     // >= max_j |c_j|^2; infinity from -kNeverWins on, or if a centroid is not finite
   uint64_t twins;                  // centroids that a later row repeats
 };
 
@@ -257,10 +262,11 @@ __device__ __forceinline__ void assign_fill(AssignLds<D, MB>& lds, const float* 
     uint64_t twins = 0ull;
     for (uint64_t m = __ballot(repeat); m; m &= m - 1)
       twins |= 1ull << __builtin_amdgcn_readlane(first, __builtin_ctzll(m));
-    const float c2max = wave_top(real ? acc : 0.0f);
+    float c2max = wave_top(real ? acc : 0.0f);
+    c2max = c2max < -kNeverWins ? c2max : INFINITY;
     if (threadIdx.x < 32 * MB) {
       lds.cn[j] = real && !repeat ? acc : INFINITY;
-      lds.a0[j] = real && !repeat ? -0.5f * acc : -1e38f;
+      lds.a0[j] = real && !repeat ? -0.5f * acc : kNeverWins;
     }
     if (threadIdx.x == 0) {
       lds.c2max = c2max;
@@ -316,9 +322,9 @@ __device__ __forceinline__ int assign_exact(const AssignLds<D, MB>& lds, const v
 }
 
 // The specification between centroids j0 < j1 of a token: lane l runs the chain
-// of j0 and lane l ^ 32 that of j1 (j: this lane's); both return the label.  A
-// NaN score never wins, and if nothing does the label is the lower one (0: only
-// centroids 0 and 1 of 2 can both be near a non-finite token).
+// of j0 and lane l ^ 32 that of j1 (j: this lane's); both return the label.
+// The token's gap is finite, so both rows are real ones (kNeverWins) and both
+// scores are finite.
 template <int D, int DT, int MB>
 __device__ __forceinline__ int assign_pair(const AssignLds<D, MB>& lds, const void* x, int64_t x0, int j) {
   const float* c = lds.cent + j * AssignLds<D, MB>::P;
@@ -337,8 +343,7 @@ __device__ __forceinline__ int assign_pair(const AssignLds<D, MB>& lds, const vo
     dot = fmaf(xv[6], c1.z, dot);
     dot = fmaf(xv[7], c1.w, dot);
   }
-  float sc = fmaf(-2.0f, dot, lds.cn[j]);
-  sc = sc < INFINITY ? sc : INFINITY;
+  const float sc = fmaf(-2.0f, dot, lds.cn[j]);
   const float so = __shfl_xor(sc, 32, 64);
   const int jo = __shfl_xor(j, 32, 64);
   return so < sc || (so == sc && jo < j) ? jo : j;

@@ -93,6 +93,29 @@ def test_repeated_centroids(gpu, s, k, dtype, pad):
         _check(x.to(dtype), gpu, k, iters=iters, seed=iters)
 
 
+@pytest.mark.parametrize("k,repeats", [(1, 0), (30, 0), (31, 0), (62, 0), (63, 0), (32, 1), (40, 1), (64, 2), (31, 5)])
+@pytest.mark.parametrize("norm2", [0.9e38, 2.2e38, 3.0e38])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_centroid_norms_near_the_top_of_fp32(gpu, k, repeats, norm2, dtype):
+    """Finite centroids whose squared norms lie on both sides of what the rows
+    that must never win (padding to a whole 32-row tile, repeats) start from,
+    and tokens short enough that no distance overflows: the label is still the
+    first smallest distance's, never a padding row or a repeat."""
+    s, h, d, seed = 20 * k + 7, 2, 128, 5
+    g = torch.Generator().manual_seed(k + repeats)
+    x = 0.02 * torch.randn(1, s, h, d, generator=g)
+    x[:, ::5] = 0.0
+    stride = s // k
+    for i in range(h):   # the rows of the initial centroids
+        c = torch.randn(k, d, generator=g, dtype=torch.float64)
+        c *= (norm2 * (0.97 + 0.06 * torch.rand(k, 1, generator=g, dtype=torch.float64))).sqrt() / c.norm(dim=1, keepdim=True)
+        c[k - repeats:] = c[0]
+        for j in range(k):
+            x[0, j * stride + okm.mix(seed, i, k, j) % stride, i] = c[j].float()
+    for iters in (1, 2, 4):
+        _check(x.to(dtype), gpu, k, iters=iters, seed=seed)
+
+
 @pytest.mark.parametrize("s,h", [(60 << 16, 2), (1024, 8192)])
 def test_noalloc_without_room_for_the_carried_state(gpu, s, h):
     """A problem that fits the built-in scratch only without the state carried
