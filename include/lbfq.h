@@ -41,6 +41,7 @@ enum {
   LBFQ_Q_CHANNEL_AMAX = 5   /* atomic max of |x| per (b,h,d) into amax_table    */
 };
 enum { LBFQ_LAYOUT_NHD = 0, LBFQ_LAYOUT_BHSD = 1, LBFQ_LAYOUT_BHDS = 2 };
+enum { LBFQ_LAYOUT_ZERO_PAD = 4 };  /* or'ed to a head-major layout: zero codes for the rows [S, codes_spitch) too */
 enum { LBFQ_DQ_BLOCK = 0, LBFQ_DQ_CHANNEL = 1, LBFQ_DQ_MX_QK = 2, LBFQ_DQ_MX_V = 3 };
 
 const char* lbfq_last_error(void);
@@ -55,7 +56,11 @@ const char* lbfq_last_error(void);
  * Per element: x[gather[s]] - sub -> round to x_dtype -> (signs, FWHT,
  * *had_scale, round) -> quantise.  One tile = R rows of one (b, h).  The
  * Hadamard rotation goes with quant modes NONE, FP8_BLOCK and MX_QK only
- * (it rotates Q/K); S and the code pitch must be below 2^31. */
+ * (it rotates Q/K); S and the code pitch must be below 2^31.  Only the S rows
+ * given are written, so a larger head-major buffer can be filled in pieces
+ * (codes advanced to the piece's first row, codes_spitch the whole extent);
+ * with LBFQ_LAYOUT_ZERO_PAD the call also clears the rows of each (b, h) from
+ * S to codes_spitch. */
 typedef struct {
   const void* x; int x_dtype;              /* input, NHD                        */
   int64_t B, S, H, D;                      /* D in {64, 128}                    */
@@ -67,8 +72,8 @@ typedef struct {
   int hadamard; const int8_t* signs;       /* signs (H, D) +-1 or NULL          */
   float had_scale;                         /* fp32(1/sqrt(D))                   */
   int quant_mode;                          /* LBFQ_Q_*                          */
-  uint8_t* codes; int codes_layout;        /* LBFQ_LAYOUT_*                     */
-  int64_t codes_spitch;                    /* S extent of BHSD/BHDS buffers; rows [S, codes_spitch) get zero codes */
+  uint8_t* codes; int codes_layout;        /* LBFQ_LAYOUT_*, with LBFQ_LAYOUT_ZERO_PAD or without */
+  int64_t codes_spitch;                    /* S extent of BHSD/BHDS buffers     */
   float* scale;                            /* scale output (see strides)        */
   int64_t sc_b, sc_s, sc_h, sc_d;          /* element strides of scale          */
   uint32_t* amax_table;                    /* (B,H,D) fp32 bits, channel modes  */

@@ -53,6 +53,7 @@ struct RowTileArgs {
   int quant_mode;
   uint8_t* codes;
   int codes_layout;
+  int zero_pad;
   int64_t codes_spitch;
   float* scale;
   int64_t sc_b, sc_s, sc_h, sc_d;
@@ -152,8 +153,9 @@ constexpr int kKeep = 4;        // resident passes per wave
 constexpr int kLB = 4;          // passes per wave in flight when streaming
 constexpr int kStageRows = 64;  // rows per BHDS staging chunk
 
-// Zero codes for the rows [S, pitch) of one (b, h): written by the workgroup of
-// its last tile, so that the buffer needs no clearing pass of its own.
+// Zero codes for the rows [S, pitch) of one (b, h) (LBFQ_LAYOUT_ZERO_PAD): written
+// by the workgroup of its last tile, so that the buffer needs no clearing pass of
+// its own.
 __device__ __forceinline__ void zero_padding(const RowTileArgs& a, int64_t bh, int tid) {
   const int64_t pad = a.codes_spitch - a.S;
   if (a.codes_layout == LBFQ_LAYOUT_BHSD) {
@@ -233,7 +235,7 @@ __device__ __forceinline__ void rowtile_body(const RowTileArgs& a, uint32_t bloc
     }
   }
   if constexpr (QM != LBFQ_Q_NONE && QM != LBFQ_Q_CHANNEL_AMAX) {
-    if (static_cast<uint32_t>(tile) + 1 == ntile && a.codes_spitch > a.S) zero_padding(a, bh, tid);
+    if (a.zero_pad && static_cast<uint32_t>(tile) + 1 == ntile && a.codes_spitch > a.S) zero_padding(a, bh, tid);
   }
   const bool sm0 = a.smoothed && a.smoothed_stage == 0, sm1 = a.smoothed && a.smoothed_stage == 1;
   __shared__ float red[kTileWaves][128];  // cross-wave reductions (D <= 128)
@@ -755,15 +757,17 @@ int rowtile_prepare(const lbfq_rowtile_params* p, RowTileLaunch* out) {
 
   LBFQ_CHECK_ARG(p->S < (1ll << 31) && p->H * p->D < (1ll << 28) && p->codes_spitch < (1ll << 31),
                  "lbfq_rowtile: S, H * D or the code pitch too large");
-  LBFQ_CHECK_ARG(p->codes_layout != LBFQ_LAYOUT_BHDS || p->codes_spitch % 4 == 0,
+  const int layout = p->codes_layout & ~LBFQ_LAYOUT_ZERO_PAD;
+  LBFQ_CHECK_ARG(layout != LBFQ_LAYOUT_BHDS || p->codes_spitch % 4 == 0,
                  "lbfq_rowtile: transposed codes pitch must be a multiple of 4");
-  LBFQ_CHECK_ARG(p->codes_layout == LBFQ_LAYOUT_NHD || p->codes_spitch >= p->S, "lbfq_rowtile: bad codes pitch");
+  LBFQ_CHECK_ARG(layout == LBFQ_LAYOUT_NHD || p->codes_spitch >= p->S, "lbfq_rowtile: bad codes pitch");
   RowTileArgs& a = out->a;
   a = RowTileArgs{};
   a.x = p->x; a.x_dtype = p->x_dtype; a.B = p->B; a.S = p->S; a.H = p->H; a.D = p->D; a.R = p->R;
   a.gather = p->gather; a.sub_mode = p->sub_mode; a.sub = p->sub; a.sub_block = p->sub_block;
   a.smoothed = p->smoothed; a.hadamard = p->hadamard; a.signs = p->signs; a.had_scale = p->had_scale;
-  a.quant_mode = qm; a.codes = p->codes; a.codes_layout = p->codes_layout; a.codes_spitch = p->codes_spitch;
+  a.quant_mode = qm; a.codes = p->codes; a.codes_layout = layout; a.codes_spitch = p->codes_spitch;
+  a.zero_pad = (p->codes_layout & LBFQ_LAYOUT_ZERO_PAD) != 0;
   a.scale = p->scale; a.sc_b = p->sc_b; a.sc_s = p->sc_s; a.sc_h = p->sc_h; a.sc_d = p->sc_d;
   a.amax_table = p->amax_table;
   a.mx_block = p->mx_block;
@@ -776,7 +780,7 @@ int rowtile_prepare(const lbfq_rowtile_params* p, RowTileLaunch* out) {
   const int64_t nblocks = ntiles;  // one workgroup per tile
   LBFQ_CHECK_ARG(nblocks < (1ll << 31), "lbfq_rowtile: grid too large");
   LBFQ_CHECK_ARG(p->R % (512 / p->D) == 0, "lbfq_rowtile: R must be a multiple of %lld", (long long)(512 / p->D));
-  out->shmem = p->codes_layout == LBFQ_LAYOUT_BHDS ? static_cast<size_t>(kStageRows * (p->D + 4)) : 0;
+  out->shmem = layout == LBFQ_LAYOUT_BHDS ? static_cast<size_t>(kStageRows * (p->D + 4)) : 0;
   out->grid = static_cast<unsigned>(nblocks);
   out->sub = p->sub_mode != LBFQ_SUB_NONE;
   out->had = p->hadamard != 0;

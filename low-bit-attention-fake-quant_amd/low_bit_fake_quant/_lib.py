@@ -21,6 +21,7 @@ DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 SUB_NONE, SUB_COLVEC, SUB_BLOCKVEC = 0, 1, 2
 Q_NONE, Q_FP8_BLOCK, Q_CHANNEL, Q_MX_QK, Q_MX_V, Q_CHANNEL_AMAX = range(6)
 LAYOUT_NHD, LAYOUT_BHSD, LAYOUT_BHDS = 0, 1, 2
+LAYOUT_ZERO_PAD = 4  # or'ed to a head-major layout
 DQ_BLOCK, DQ_CHANNEL, DQ_MX_QK, DQ_MX_V = range(4)
 
 _i64 = ctypes.c_int64

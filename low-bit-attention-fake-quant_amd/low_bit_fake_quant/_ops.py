@@ -43,7 +43,10 @@ def rowtile_params(src: RowSource, *, R: int, smoothed: torch.Tensor | None = No
                    signs: torch.Tensor | None = None, hadamard: bool = False, had_scale: float = 1.0,
                    quant_mode: int = _lib.Q_NONE, codes: torch.Tensor | None = None, codes_layout: int = _lib.LAYOUT_NHD,
                    codes_spitch: int = 0, scale: torch.Tensor | None = None, scale_strides=(0, 0, 0, 0),
-                   amax_table: torch.Tensor | None = None, mx_block: int = 32, scale_e8m0: bool = False) -> _lib.RowTileParams:
+                   amax_table: torch.Tensor | None = None, mx_block: int = 32, scale_e8m0: bool = False,
+                   zero_pad: bool = True) -> _lib.RowTileParams:
+    """zero_pad: the call clears rows [S, codes_spitch) of head-major codes (off
+    for a call that fills a piece of a larger buffer)."""
     x = src.x
     b, s, h, d = x.shape
     p = _lib.RowTileParams()
@@ -55,7 +58,8 @@ def rowtile_params(src: RowSource, *, R: int, smoothed: torch.Tensor | None = No
     p.smoothed = _lib.ptr(smoothed)
     p.hadamard = 1 if hadamard else 0; p.signs = _lib.ptr(signs); p.had_scale = float(had_scale)
     p.quant_mode = quant_mode
-    p.codes = _lib.ptr(codes); p.codes_layout = codes_layout; p.codes_spitch = int(codes_spitch)
+    p.codes = _lib.ptr(codes); p.codes_layout = codes_layout | (_lib.LAYOUT_ZERO_PAD if zero_pad else 0)
+    p.codes_spitch = int(codes_spitch)
     p.scale = _lib.ptr(scale)
     p.sc_b, p.sc_s, p.sc_h, p.sc_d = (int(v) for v in scale_strides)
     p.amax_table = _lib.ptr(amax_table)

@@ -155,6 +155,25 @@ def test_rowtile_rejects_hadamard_with_v_modes():
         assert b"Hadamard" in lib.lbfq_last_error()
 
 
+def test_rowtile_checks_the_pitch_with_and_without_the_padding_flag():
+    """The pitch checks of the head-major layouts hold whether the padding rows
+    are asked for or not (host-side checks, no GPU needed)."""
+    from low_bit_fake_quant import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built (run __graft_entry__.build())")
+    lib = _lib.load(require_gpu=False)
+    for flag in (0, _lib.LAYOUT_ZERO_PAD):
+        for layout, qm, pitch, msg in ((_lib.LAYOUT_BHDS, _lib.Q_CHANNEL, 258, b"multiple of 4"),
+                                       (_lib.LAYOUT_BHDS, _lib.Q_CHANNEL, 252, b"bad codes pitch"),
+                                       (_lib.LAYOUT_BHSD, _lib.Q_FP8_BLOCK, 192, b"bad codes pitch")):
+            p = _lib.RowTileParams()
+            p.x = 0x1000; p.x_dtype = 2; p.B, p.S, p.H, p.D = 1, 256, 2, 128; p.R = 64
+            p.quant_mode = qm; p.codes = 0x2000; p.codes_layout = layout | flag; p.codes_spitch = pitch
+            p.scale = 0x3000; p.amax_table = 0x4000; p.mx_block = 32
+            assert lib.lbfq_rowtile(p, None) != 0
+            assert msg in lib.lbfq_last_error()
+
+
 def test_sdpa_entry_points_reject_bad_arguments_without_a_gpu():
     """lbfq_sdpa_dequant / lbfq_sdpa_fwd validate their parameters before any
     HIP call: bad parameters return -1 with a message, with no device present.
