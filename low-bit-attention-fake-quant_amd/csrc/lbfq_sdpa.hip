@@ -665,13 +665,14 @@ __global__ void __launch_bounds__(NW * 64, 2) sdpa_split_kernel(const SdpaArgs a
       float tmax = u[0];
 #pragma unroll
       for (int j = 1; j < 32; ++j) tmax = fmaxf(tmax, u[j]);
-      const float m_new = fmaxf(m, xor32_max(tmax));  // finite: key 64 t is valid
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 0 on the wave's first tile
+      const float m_new = fmaxf(m, xor32_max(tmax));
+      const float ms = m_new == -INFINITY ? 0.0f : m_new;  // the wave's products so far all overflowed
+      const float alpha = __builtin_amdgcn_exp2f(m - ms);  // 0 on the wave's first tile
       m = m_new;
       float sum = 0.0f;
 #pragma unroll
       for (int j = 0; j < 32; ++j) {
-        u[j] = __builtin_amdgcn_exp2f(u[j] - m_new);
+        u[j] = __builtin_amdgcn_exp2f(u[j] - ms);
         sum += u[j];
       }
       l = l * alpha + sum;
