@@ -340,7 +340,10 @@ class _SimBf16(_Sim):
     rows, v as (H, D, S)."""
 
     def operand(self, x3, *, quantise: bool, transposed: bool):
-        """(operand, QuantStats or None) of an (S, H, D) tensor."""
+        """(operand, QuantStats or None) of an (S, H, D) tensor; unquantised, of
+        any dtype that casts to bf16."""
+        if not quantise and x3.dtype not in _lib.DTYPE_CODE:
+            x3 = x3.to(torch.bfloat16)
         x3 = x3.contiguous()
         if x3.dtype not in _lib.DTYPE_CODE:
             raise TypeError(f"unsupported dtype {x3.dtype}")

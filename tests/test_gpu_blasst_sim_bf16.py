@@ -55,3 +55,17 @@ def test_one_tensor_as_all_three(gpu):
     for lv in one.outputs:
         assert torch.equal(one.outputs[lv], three.outputs[lv])
     _close(one.outputs["bf16_ref"][0].cpu(), osim.simulate(x, x, x)["bf16_ref"])
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.int32])
+def test_reference_rung_takes_any_dtype_that_casts(gpu, dtype):
+    """The bf16 reference rung rounds its operands to bf16 whatever they are;
+    the quantising rungs take the float dtypes of the kernels only."""
+    from low_bit_fake_quant import blasst_skip as bs
+    q, k, v = ((3 * cpu_randn(1, 256, 2, 64, seed=i, dtype=torch.float64)).to(dtype).to(gpu) for i in range(3))
+    res = bs.simulate_workload(q, k, v, skip_thresholds=[], levels=[bs.LEVEL_REFERENCE])
+    want = bs.simulate_workload(*(t.to(torch.bfloat16) for t in (q, k, v)), skip_thresholds=[],
+                                levels=[bs.LEVEL_REFERENCE])
+    assert torch.equal(res.outputs[bs.LEVEL_REFERENCE], want.outputs[bs.LEVEL_REFERENCE])
+    with pytest.raises(TypeError, match="unsupported dtype"):
+        bs.simulate_workload(q, k, v, skip_thresholds=[], levels=[bs.LEVEL_FP8_QKV])
