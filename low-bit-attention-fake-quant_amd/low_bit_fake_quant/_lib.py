@@ -227,11 +227,14 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # private: builds may lack it
+
+
 def stream_handle(device=None) -> int:
     """The hipStream_t of torch's current stream on ``device``.  Tensors' devices
     carry an index, which torch resolves to the raw handle directly (0.2 us;
     building its Stream object takes 3)."""
     index = getattr(device, "index", None)
-    if index is None:
+    if index is None or _raw_stream is None:
         return torch.cuda.current_stream(device).cuda_stream
-    return torch._C._cuda_getCurrentRawStream(index)
+    return _raw_stream(index)

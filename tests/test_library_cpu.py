@@ -174,6 +174,22 @@ def test_rowtile_checks_the_pitch_with_and_without_the_padding_flag():
             assert msg in lib.lbfq_last_error()
 
 
+def test_stream_handle_without_torchs_private_call(monkeypatch):
+    """The current stream's handle comes from torch's private raw-stream call
+    where the device has an index, and from the public API in a torch without
+    that call or for a device without an index."""
+    from types import SimpleNamespace
+
+    from low_bit_fake_quant import _lib
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: SimpleNamespace(cuda_stream=("public", d)))
+    monkeypatch.setattr(_lib, "_raw_stream", lambda i: ("raw", i))
+    dev, bare = torch.device("cuda", 1), torch.device("cuda")
+    assert _lib.stream_handle(dev) == ("raw", 1)
+    assert _lib.stream_handle(bare) == ("public", bare)
+    monkeypatch.setattr(_lib, "_raw_stream", None)
+    assert _lib.stream_handle(dev) == ("public", dev)
+
+
 def test_sdpa_entry_points_reject_bad_arguments_without_a_gpu():
     """lbfq_sdpa_dequant / lbfq_sdpa_fwd validate their parameters before any
     HIP call: bad parameters return -1 with a message, with no device present.
