@@ -410,14 +410,20 @@ __global__ void __launch_bounds__(64) attend_kernel(const float* q, const float*
 // The row's final max is known from the scan, so nothing is rescaled.
 //
 // At 8 heads x 16384 x 128 (0.55 TFLOP a product) the scan takes 0.51 ms, the
-// exact and online rungs 1.45 and 1.54, static P 1.8 (2.4 with its statistics,
+// exact and online rungs 1.40 and 1.47, static P 1.73 (2.4 with its statistics,
 // whose squared errors are fp64): 1.1 PFLOP/s in the scan, which the MFMAs and
 // their LDS reads bound, and 0.6-0.8 in the rungs, which the exponentials and
 // conversions bound. The fp32 kernels, bound by FMA issue, took 11, 57, 57
-// and 70 ms on the same operands. Error against 64-bit arithmetic, mean over 16
-// draws of 1024 to 8192 tokens: 7.0e-6 in the bf16 rung (1.05e-5 there), 1.1e-5
-// (1.2e-5) with FP8 operands and 2.5e-5 (2.4e-5) with FP8 P, where the few P that
-// round the other way make most of it on both sides.
+// and 70 ms on the same operands.
+//
+// The weights are formed from differences of the unscaled scores, which lie
+// close together and so differ without a rounding, with sm log2 e as the
+// exponent's factor: a score scaled first is off by 2^-24 of itself, as much as
+// the products' own error. Mean error of a head against 64-bit arithmetic, 6000
+// heads of 1024 and 2048 tokens x 128: 9.2e-6 in the bf16 rung (the fp32 kernels
+// 9.2e-6), 9.3e-6 (9.4e-6) with FP8 operands and 1.9e-5 (2.0e-5) with FP8 P;
+// scaled first 9.4e-6, 9.6e-6 and 2.0e-5. The FP8 P that round the other way, of
+// 3.7e9: 17.5e3 (18.8e3; scaled first 19.1e3).
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -453,15 +459,25 @@ __device__ __forceinline__ float pair_add(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// F exp(x) for x <= 0, F a power of two: exp2 of the rounded product x log2 e,
-// corrected to first order for what the rounding and log2 e's own low part
-// leave out (v_exp_f32 is good to 1 ulp, the rounded product alone is off by
-// |x| 2^-24).
+// F exp(c x / log2 e) for x <= 0, c = hi + lo > 0 and F a power of two: exp2 of the
+// rounded product x hi, corrected to first order for what the rounding and c's
+// low part leave out (v_exp_f32 is good to 1 ulp, the rounded product alone is
+// off by |x c| 2^-24).
+struct ExpFactor {
+  float hi, lo;
+};
+// log2 e, and sm log2 e for differences of unscaled scores
+constexpr ExpFactor kLog2e = {1.44269502f, 1.92596303e-8f};
+__device__ __forceinline__ ExpFactor exp_factor(float sm) {
+  const double c = static_cast<double>(sm) * 1.4426950408889634;
+  const float hi = static_cast<float>(c);
+  return {hi, static_cast<float>(c - static_cast<double>(hi))};
+}
 template <int F>
-__device__ __forceinline__ float exp_scaled(float x) {
-  constexpr float kL = 1.44269502f, kLo = 1.92596303e-8f, kLn2 = 0.693147182f;
-  const float t = x * kL;
-  const float lo = fmaf(x, kLo, fmaf(x, kL, -t));
+__device__ __forceinline__ float exp_scaled(float x, ExpFactor c) {
+  constexpr float kLn2 = 0.693147182f;
+  const float t = x * c.hi;
+  const float lo = fmaf(x, c.lo, fmaf(x, c.hi, -t));
   const float e = __builtin_amdgcn_exp2f(t) * static_cast<float>(F);
   const float r = fmaf(e, lo * kLn2, e);
   return e == 0.0f ? 0.0f : r;  // x = -inf: lo is not a number
@@ -608,7 +624,8 @@ __global__ void __launch_bounds__(kMmThreads, 2)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
   // den, tot_l, drop_l: this lane's keys; the lane pair's are added at the end
-  float den = 0.0f, tot_l = 0.0f, drop_l = 0.0f, rm = -INFINITY;
+  float den = 0.0f, tot_l = 0.0f, drop_l = 0.0f, mu = -INFINITY;  // mu: the running max, unscaled
+  const ExpFactor ef = exp_factor(sm_scale);
   unsigned uf = 0;  // at most 64 keys of S / 128 blocks
   double sq = 0.0;
   u32x4 kr[St::CH], vr[St::CH];
@@ -622,12 +639,11 @@ __global__ void __launch_bounds__(kMmThreads, 2)
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) s[kb] = mm_scores<D, true>(buf, kb, li, g, qop);
     mm_load<D, true>(kh, vh, S, (j + 1 < nb ? j + 1 : j) * kTileQ, tid, kr, vr);
-    float ref = fm, rescale = 1.0f;
+    float rescale = 1.0f;
     if constexpr (MODE != 0) {
       const float m = fmaxf(fmaxf(max16(s[0]), max16(s[1])), fmaxf(max16(s[2]), max16(s[3])));
-      rm = fmaxf(rm, pair_max(m) * sm_scale);
-      ref = rm;
-      rescale = exp_scaled<1>(rm - fm);
+      mu = fmaxf(mu, pair_max(m));
+      rescale = exp_scaled<1>(mu * sm_scale - fm, kLog2e);
     }
     // a skipped block adds nothing; its unquantised mass is still needed for
     // the dropped-mass diagnostic and the P statistics cover all blocks
@@ -642,11 +658,11 @@ __global__ void __launch_bounds__(kMmThreads, 2)
         for (int r = 0; r < 16; r += 2) {
           float p[2];
           if constexpr (MODE == 2) {
-            float x[2], sc[2];  // s - rm, 256 exp(s - rm)
+            float x[2], sc[2];  // the unscaled difference to the running max, 256 exp of the scaled one
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-              x[e] = s[kb][r + e] * sm_scale - ref;
-              sc[e] = exp_scaled<256>(x[e]);
+              x[e] = s[kb][r + e] - mu;
+              sc[e] = exp_scaled<256>(x[e], ef);
               lb += sc[e];
             }
             const int code = __builtin_amdgcn_cvt_pk_fp8_f32(sc[0], sc[1], 0, false);
@@ -657,7 +673,7 @@ __global__ void __launch_bounds__(kMmThreads, 2)
               if constexpr (STATS) {
                 const float on = sc[e] * (1.0f / 256.0f), err = d * (1.0f / 256.0f) - on;  // exact difference
                 // exp(x) > 0 down to the smallest denormal, below what v_exp_f32 returns
-                uf += static_cast<unsigned>(d == 0.0f) & static_cast<unsigned>(x[e] > -103.972077f);
+                uf += static_cast<unsigned>(d == 0.0f) & static_cast<unsigned>(x[e] * sm_scale > -103.972077f);
                 sq += static_cast<double>(err) * static_cast<double>(err);
               }
               p[e] = d * rs;
@@ -665,8 +681,8 @@ __global__ void __launch_bounds__(kMmThreads, 2)
           } else {
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-              p[e] = exp_scaled<1>(s[kb][r + e] * sm_scale - ref);
-              if constexpr (MODE == 1) p[e] *= rescale;
+              if constexpr (MODE == 1) p[e] = exp_scaled<1>(s[kb][r + e] - mu, ef) * rescale;
+              else p[e] = exp_scaled<1>(fmaf(s[kb][r + e], sm_scale, -fm), kLog2e);
               lb += p[e];
             }
           }

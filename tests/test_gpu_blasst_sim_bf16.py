@@ -69,3 +69,33 @@ def test_reference_rung_takes_any_dtype_that_casts(gpu, dtype):
     assert torch.equal(res.outputs[bs.LEVEL_REFERENCE], want.outputs[bs.LEVEL_REFERENCE])
     with pytest.raises(TypeError, match="unsupported dtype"):
         bs.simulate_workload(q, k, v, skip_thresholds=[], levels=[bs.LEVEL_FP8_QKV])
+
+
+@pytest.mark.parametrize("mode,lv", [(1, "fp8_qkv"), (2, "fp8_static_p")])
+@pytest.mark.parametrize("d", [64, 128])
+def test_large_scores_keep_their_differences(gpu, d, mode, lv):
+    """Scores that are exact integers around 13000: the weights depend on their
+    differences, which are exact, so a rung is within fp32 exponentials and sums
+    of 64 bits (rounding each scaled score would put 2^-24 * 13000 / sqrt(d) =
+    1e-4 on each weight, and a thousandth of them on another E4M3 code)."""
+    from low_bit_fake_quant import blasst_skip as bs
+    s, h = 128, 16   # one block: its maximum is the final one
+    g = torch.Generator().manual_seed(d + mode)
+    q, k = (torch.randint(-2, 3, (s, h, d), generator=g).float() for _ in range(2))
+    q[..., 0], k[..., 0] = 64.0, 200.0
+    v = torch.randn(s, h, d, generator=g).to(torch.bfloat16)
+    sim = bs._SimBf16(s, h, d, d ** -0.5, gpu)
+    qg, kg, vg = (sim.operand(t.to(torch.bfloat16).to(gpu), quantise=False, transposed=tr)[0]
+                  for t, tr in ((q, False), (k, False), (v, True)))
+    fm = sim.scan(qg, kg)[0]
+    out = sim.attend(qg, kg, vg, fm, mode, True)[0].cpu().double().permute(1, 0, 2)
+    qd, kd, vd = (t.double().permute(1, 0, 2) for t in (q, k, v))
+    u = qd @ kd.transpose(1, 2)
+    top = u.amax(-1, keepdim=True)
+    sm = float(torch.tensor(d ** -0.5, dtype=torch.float32))   # the scale the kernels are given
+    p = torch.exp((u - top) * sm)
+    w = (p * 256.0).float().to(torch.float8_e4m3fn).double() / 256.0 if mode == 2 else p
+    want = w.to(torch.bfloat16).double() @ vd / p.sum(-1, keepdim=True)
+    # fp32 sums and quotients stay within 2^-20; the few weights within 2^-22 of a rounding boundary may fall on
+    # the other side of it (of 2^18 weights about one, by 2^-4 of a single weight)
+    assert float((out - want).norm() / want.norm()) <= 2e-5
