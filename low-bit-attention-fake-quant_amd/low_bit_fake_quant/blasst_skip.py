@@ -193,28 +193,26 @@ def _check_gpu(x: torch.Tensor, what: str) -> None:
         raise ValueError(f"{what} requires CUDA tensors")
 
 
-def _head_quant(x3: torch.Tensor, mm_dtype: Optional[torch.dtype], want_deq: bool):
-    """(deq fp32 or None, deq rounded to mm_dtype as fp32 or None, scale (H,), QuantStats)."""
+def _head_quant(x3: torch.Tensor):
+    """(deq fp32, scale (H,), QuantStats)."""
     s, h, d = x3.shape
     x3 = x3.contiguous()
     if x3.dtype not in _lib.DTYPE_CODE:
         raise TypeError(f"unsupported dtype {x3.dtype}")
     dev = x3.device
-    deq = torch.empty(s, h, d, dtype=torch.float32, device=dev) if want_deq else None
-    deq_mm = torch.empty(s, h, d, dtype=torch.float32, device=dev) if mm_dtype is not None else None
+    deq = torch.empty(s, h, d, dtype=torch.float32, device=dev)
     scale = torch.empty(h, dtype=torch.float32, device=dev)
     ws = torch.empty(h, dtype=torch.int32, device=dev)
     counts = torch.zeros(2, dtype=torch.int64, device=dev)
     sqerr = torch.zeros(1, dtype=torch.float64, device=dev)
     lib = _lib.load()
-    _lib.check(lib.lbfq_head_fp8_quant(x3.data_ptr(), _lib.DTYPE_CODE[x3.dtype], s, h, d, _lib.ptr(deq),
-                                       _lib.ptr(deq_mm), int(mm_dtype == torch.bfloat16), scale.data_ptr(),
-                                       ws.data_ptr(), counts.data_ptr(), sqerr.data_ptr(),
+    _lib.check(lib.lbfq_head_fp8_quant(x3.data_ptr(), _lib.DTYPE_CODE[x3.dtype], s, h, d, deq.data_ptr(), None, 0,
+                                       scale.data_ptr(), ws.data_ptr(), counts.data_ptr(), sqerr.data_ptr(),
                                        _lib.stream_handle(dev)), "head_fp8_quant")
     n = x3.numel()
     c = counts.tolist()
     stats = QuantStats(c[0] / n, c[1] / n, math.sqrt(float(sqerr.item()) / n))
-    return deq, deq_mm, scale, stats
+    return deq, scale, stats
 
 
 def fake_quant_per_head(x: torch.Tensor):
@@ -223,7 +221,7 @@ def fake_quant_per_head(x: torch.Tensor):
     if x.ndim != 3:
         raise ValueError(f"expected (S, H, D); got {tuple(x.shape)}")
     _check_gpu(x, "fake_quant_per_head")
-    deq, _, scale, stats = _head_quant(x, None, True)
+    deq, scale, stats = _head_quant(x)
     return deq, scale.view(1, -1, 1), stats
 
 
@@ -316,7 +314,7 @@ class _Sim:
                    "blasst_keep")
         return keep, counts.tolist()
 
-    def attend(self, q, k, v, fm, mode, round_p, keep=None, dropped=False, p_stats=False):
+    def attend(self, q, k, v, fm, mode, keep=None, dropped=False, p_stats=False):
         out = torch.empty(self.s, self.h, self.d, dtype=torch.float32, device=self.dev)
         drop = torch.empty(self.h, self.s, dtype=torch.float32, device=self.dev) if dropped else None
         pc = torch.zeros(2, dtype=torch.int64, device=self.dev) if p_stats else None
@@ -325,7 +323,7 @@ class _Sim:
         p.S, p.H, p.D = self.s, self.h, self.d
         p.q, p.k, p.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
         p.sm_scale = self.sm
-        p.mode, p.round_p_bf16 = mode, int(round_p)
+        p.mode = mode  # P stays fp32, as the operands
         p.final_max = fm.data_ptr()
         p.keep = _lib.ptr(keep)
         p.out = out.data_ptr()
@@ -373,7 +371,7 @@ class _SimBf16(_Sim):
                    "blasst_scan_bf16")
         return fm, tm, tb
 
-    def attend(self, q, k, v, fm, mode, round_p, keep=None, dropped=False, p_stats=False):
+    def attend(self, q, k, v, fm, mode, keep=None, dropped=False, p_stats=False):
         out = torch.empty(self.s, self.h, self.d, dtype=torch.float32, device=self.dev)
         drop = torch.empty(self.h, self.s, dtype=torch.float32, device=self.dev) if dropped else None
         pc = torch.zeros(2, dtype=torch.int64, device=self.dev) if p_stats else None
@@ -415,7 +413,6 @@ def simulate_workload(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, skip
     thresholds = list(skip_thresholds)
     want_skip = LEVEL_FP8_SKIP in levels and len(thresholds) > 0
     want_fp8 = any(lv in levels for lv in (LEVEL_FP8_QKV, LEVEL_FP8_STATIC_P, LEVEL_FP8_SKIP))
-    round_p = matmul_dtype == torch.bfloat16
     dev = q.device
     on_mfma = matmul_dtype == torch.bfloat16
     sim = (_SimBf16 if on_mfma else _Sim)(s, h, d, 1.0 / math.sqrt(d), dev)
@@ -427,9 +424,9 @@ def simulate_workload(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, skip
             qr, kr, vr = (sim.operand(t[0], quantise=False, transposed=tr)[0]
                           for t, tr in ((q, False), (k, False), (v, True)))
         else:
-            qr, kr, vr = (t[0].to(matmul_dtype).float().contiguous() for t in (q, k, v))
+            qr, kr, vr = (t[0].float().contiguous() for t in (q, k, v))
         fm, _, _ = sim.scan(qr, kr)
-        out, *_ = sim.attend(qr, kr, vr, fm, 0, round_p)
+        out, *_ = sim.attend(qr, kr, vr, fm, 0)
         result.outputs[LEVEL_REFERENCE] = out.view(1, s, h, d)
         del qr, kr, vr, fm
 
@@ -439,17 +436,17 @@ def simulate_workload(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, skip
             if on_mfma:
                 mm, st = sim.operand(t[0], quantise=True, transposed=name == "v")
             else:
-                _, mm, _, st = _head_quant(t[0], matmul_dtype, False)
+                mm, _, st = _head_quant(t[0])
             dst.append(mm)
             result.quant_stats[name] = st
         qd, kd, vd = qd[0], kd[0], vd[0]
         fm, tm, tb = sim.scan(qd, kd)
         if LEVEL_FP8_QKV in levels:
-            out, *_ = sim.attend(qd, kd, vd, fm, 1, round_p)
+            out, *_ = sim.attend(qd, kd, vd, fm, 1)
             result.outputs[LEVEL_FP8_QKV] = out.view(1, s, h, d)
         p_stats_done = False
         if LEVEL_FP8_STATIC_P in levels:
-            out, _, pc, pe = sim.attend(qd, kd, vd, fm, 2, round_p, p_stats=True)
+            out, _, pc, pe = sim.attend(qd, kd, vd, fm, 2, p_stats=True)
             result.outputs[LEVEL_FP8_STATIC_P] = out.view(1, s, h, d)
             p_stats_done = True
         if want_skip:
@@ -457,7 +454,7 @@ def simulate_workload(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, skip
             total_pairs = (s // QUERY_TILE) * h * sim.nb
             for i, th in enumerate(thresholds):
                 stats_here = not p_stats_done and i == 0
-                out, drop, pc_i, pe_i = sim.attend(qd, kd, vd, fm, 2, round_p, keep=keep[i],
+                out, drop, pc_i, pe_i = sim.attend(qd, kd, vd, fm, 2, keep=keep[i],
                                                    dropped=collect_dropped_mass, p_stats=stats_here)
                 if stats_here:
                     pc, pe = pc_i, pe_i

@@ -88,7 +88,7 @@ def test_large_scores_keep_their_differences(gpu, d, mode, lv):
     qg, kg, vg = (sim.operand(t.to(torch.bfloat16).to(gpu), quantise=False, transposed=tr)[0]
                   for t, tr in ((q, False), (k, False), (v, True)))
     fm = sim.scan(qg, kg)[0]
-    out = sim.attend(qg, kg, vg, fm, mode, True)[0].cpu().double().permute(1, 0, 2)
+    out = sim.attend(qg, kg, vg, fm, mode)[0].cpu().double().permute(1, 0, 2)
     qd, kd, vd = (t.double().permute(1, 0, 2) for t in (q, k, v))
     u = qd @ kd.transpose(1, 2)
     top = u.amax(-1, keepdim=True)
@@ -99,3 +99,40 @@ def test_large_scores_keep_their_differences(gpu, d, mode, lv):
     # fp32 sums and quotients stay within 2^-20; the few weights within 2^-22 of a rounding boundary may fall on
     # the other side of it (of 2^18 weights about one, by 2^-4 of a single weight)
     assert float((out - want).norm() / want.norm()) <= 2e-5
+
+
+def test_fp32_entries_with_bf16_rounding(gpu):
+    """The C entries of the fp32 kernels round their operands (mm_bf16) and P
+    (round_p_bf16) to bf16 where asked: the rungs of the matrix-core entries."""
+    from low_bit_fake_quant import _lib as L
+    from low_bit_fake_quant import blasst_skip as bs
+    s, h, d = 384, 2, 64
+    xs = [cpu_randn(s, h, d, seed=60 + i).to(gpu) for i in range(3)]
+    lib, st = L.load(), L.stream_handle(gpu)
+
+    def quantised(x):
+        deq, mm = (torch.empty(s, h, d, device=gpu) for _ in range(2))
+        scale, ws = torch.empty(h, device=gpu), torch.empty(h, dtype=torch.int32, device=gpu)
+        counts, sq = torch.zeros(2, dtype=torch.int64, device=gpu), torch.zeros(1, dtype=torch.float64, device=gpu)
+        L.check(lib.lbfq_head_fp8_quant(x.data_ptr(), L.DTYPE_CODE[x.dtype], s, h, d, deq.data_ptr(), mm.data_ptr(), 1,
+                                        scale.data_ptr(), ws.data_ptr(), counts.data_ptr(), sq.data_ptr(), st), "quant")
+        assert torch.equal(mm, deq.to(torch.bfloat16).float())
+        return mm
+
+    fp32, mfma = bs._Sim(s, h, d, d ** -0.5, gpu), bs._SimBf16(s, h, d, d ** -0.5, gpu)
+    a = [quantised(x) for x in xs]
+    b = [mfma.operand(x, quantise=True, transposed=i == 2)[0] for i, x in enumerate(xs)]
+    assert torch.equal(a[0].permute(1, 0, 2), b[0].float()) and torch.equal(a[2].permute(1, 2, 0), b[2].float())
+    fm = fp32.scan(a[0], a[1])[0]
+    for mode in (0, 1, 2):
+        out = torch.empty(s, h, d, device=gpu)
+        p = L.BlasstAttendParams()
+        p.S, p.H, p.D = s, h, d
+        p.q, p.k, p.v = (t.data_ptr() for t in a)
+        p.sm_scale, p.mode, p.round_p_bf16, p.final_max, p.out = d ** -0.5, mode, 1, fm.data_ptr(), out.data_ptr()
+        L.check(lib.lbfq_blasst_attend(p, st), "attend")
+        plain = fp32.attend(*a, fm, mode)[0]
+        want = mfma.attend(*b, mfma.scan(b[0], b[1])[0], mode)[0]
+        _close(out.cpu(), want.cpu())
+        # rounded, unlike P in fp32 (in the static rung the online weights' codes are bf16 values but for the rescale)
+        assert mode == 2 or float((out - want).norm()) < 0.2 * float((plain - want).norm())
