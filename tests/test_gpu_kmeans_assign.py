@@ -137,3 +137,31 @@ def test_noalloc_without_room_for_the_carried_state(gpu, s, h):
     torch.cuda.synchronize()
     for got, want in zip(*outs):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("spread", [0, 4, 12])
+@pytest.mark.parametrize("carry", [False, True])
+def test_mfma_error_that_the_gap_allows_for(gpu, carry, spread):
+    """The assignment's gap counts 2^-20 of the magnitudes added for each
+    v_mfma_f32_32x32x16_bf16.  One such instruction, its accumulator zero or
+    (carry) one product of an earlier one, through the simulator's score scan
+    at scale 1: every key of a head is the same, so a row's maximum is its
+    score.  Operands of one magnitude up to ones over 2^24 (products 2^48)."""
+    from low_bit_fake_quant.blasst_skip import _SimBf16
+    s, h, d = 128, 256, 64
+    g = torch.Generator().manual_seed(spread + 100 * carry)
+
+    def values(*shape):
+        mag = torch.exp2(spread * (2 * torch.rand(*shape, generator=g) - 1))
+        return (torch.randn(*shape, generator=g) * mag).to(torch.bfloat16)
+
+    q, k = torch.zeros(h, s, d, dtype=torch.bfloat16), torch.zeros(h, 1, d, dtype=torch.bfloat16)
+    q[..., 16:32], k[..., 16:32] = values(h, s, 16), values(h, 1, 16)
+    if carry:   # dimensions 0-15 come first: one exact product stands in the accumulator
+        q[..., 0], k[..., 0] = 8 * values(h, s), values(h, 1)
+    sim = _SimBf16(s, h, d, 1.0, gpu)
+    got = sim.scan(q.to(gpu), k.expand(h, s, d).contiguous().to(gpu))[0].cpu().double()
+    prod = q.double() * k.double()
+    worst = float(((got - prod.sum(-1)).abs() / prod.abs().sum(-1).clamp_min(1e-300)).max())
+    print(f"largest MFMA error / magnitudes, spread 2^{spread}, carry {carry}: {worst * 2 ** 20:.3f} * 2^-20")
+    assert worst <= 2.0 ** -20
