@@ -169,14 +169,15 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& 
 // they doubled the kernel's time).  Any more, and one lane per centroid runs
 // the chains at once.
 //
-// At 40 x 32768 x 128 bf16 (335 MB, 62 us as reads alone in this pattern) a
-// full round takes 118 us with 32 clusters and 105 with 64; one token per lane
-// against LDS broadcasts, bound by its FMA issue, took 196 and 345.  The rest
-// is ~27 us of latency before the first tokens (centroids, bounds, lists),
-// which is also what a late round with few open tokens takes.  A step issues
-// three VALU instructions per centroid and token pair of lanes (number in,
-// second, first); with separate passes for the maximum, the near mask and the
-// runner-up it issued eight and took 121 us with 64 clusters.
+// At 40 x 32768 x 128 bf16 (335 MB, 62 us as reads alone in this pattern) the
+// first round takes 112 us with 32 clusters, and a full one 108 to 122 with 64;
+// one token per lane against LDS broadcasts, bound by its FMA issue, took 196
+// and 345.  The rest is latency before the first tokens (centroids, bounds,
+// lists), and that is what a late round with few open tokens takes: 28 us there,
+// 13 at 12 x 8192.  A step issues three VALU instructions per centroid and token
+// pair of lanes (number in, second, first); with separate passes for the
+// maximum, the near mask and the runner-up it issued eight and took 15% longer
+// with 64 clusters.
 constexpr int kAsgWaves = 8;
 constexpr int kAsgThreads = 64 * kAsgWaves;
 constexpr int kSlab = 32 * kAsgWaves;  // tokens per slab: one 32-token step of each wave
@@ -657,13 +658,14 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
 // unless more than a quarter of the chunk moved.
 //
 // Bound by the row reads and the LDS sort ahead of them: at 40 x 32768 x 128
-// bf16 with 32 clusters the first round (the ranges included) takes 97 us, the
-// later ones 60, 25, 18, then 15 as fewer tokens move; with 64 clusters 119, 83,
-// 52, then 45 to 35 (16 lanes to a cluster: 125, 67, 31, 18, 14, and every
+// bf16 with 32 clusters the first round (the ranges included) takes 90 us, the
+// later ones 58, 24, 17, then 16 to 14 as fewer tokens move; with 64 clusters 113,
+// 83, 54, then 47 to 39 (16 lanes to a cluster: 125, 67, 31, 18, 14, and every
 // round 132 us with one column and a 2-byte load per lane and no moves).
 //
 // Where one chunk is the slice, `cent` is not null and the centroids follow at
-// once: with a pass of its own ten rounds over 2 x 512 x 128 take 366 us, 295 so.
+// once: with a pass of its own ten rounds over 2 x 512 x 128 (272 tokens and
+// padding) take 387 us, 303 so.
 constexpr int kUpdThreads = 512;
 constexpr int kMaxMoved = kChunk / 4;
 
