@@ -361,8 +361,16 @@ __device__ __forceinline__ int assign_pair(const AssignLds<D, MB>& lds, const vo
 // further apart than twice the error of the specification's fp32 scores
 // (2^-16 X C + 2^-17 C^2 each, X <= u + C), the label is what the
 // specification would choose again, and the token's row is not read.  All
-// roundings are taken outwards by 2^-18 relative, 50 times their size.
+// roundings are taken outwards by 2^-18 relative, 50 times their size; the sums
+// over the rounds, however many, are rounded up as they grow (add_up), so that
+// no difference of two of them is short of the path between.
 constexpr float kOut = 0x1p-18f;
+
+// a + b or more, for a, b >= 0 (a step below half a last bit of the path so far counts too)
+__device__ __forceinline__ float add_up(float a, float b) {
+  const float s = a + b;
+  return fmaf(s, 0x1p-22f, s);
+}
 
 // label still certain: (st.x, st.y) the stored pair, cum and cmax of now, c >= max_j |c_j|
 __device__ __forceinline__ bool bounds_hold(float2 st, float cum, float cmax, float c) {
@@ -420,7 +428,7 @@ __global__ void __launch_bounds__(kAsgThreads, 4)
         if (static_cast<int>(threadIdx.x) < K) cum_s[threadIdx.x] = tr.cum[bh * K + threadIdx.x];
         cmax = 0.0f;
         if (prev_changed)
-          cmax = tr.cum_max[(it & 1) * BH + bh] + wave_top(lane < K ? tr.delta[bh * K + lane] : 0.0f);
+          cmax = add_up(tr.cum_max[(it & 1) * BH + bh], wave_top(lane < K ? tr.delta[bh * K + lane] : 0.0f));
         if (s_in == 0 && threadIdx.x == 0) tr.cum_max[((it + 1) & 1) * BH + bh] = cmax;
         __syncthreads();
       }
@@ -813,7 +821,7 @@ __global__ void __launch_bounds__(kUpdThreads, 8) km_update_partial_kernel(const
       if (lane == 0) {
         const float step = step_length(s);
         tr.delta[bh * K + j] = step;
-        tr.cum[bh * K + j] += step;
+        tr.cum[bh * K + j] = add_up(tr.cum[bh * K + j], step);
       }
     }
   };
@@ -987,7 +995,7 @@ __global__ void __launch_bounds__(D) km_finalize_kernel(const double* partial, c
       if (D == 128) s += red[1];
       const float step = step_length(s);
       tr.delta[bh * K + j] = step;
-      tr.cum[bh * K + j] += step;
+      tr.cum[bh * K + j] = add_up(tr.cum[bh * K + j], step);
       tr.touched[bh * K + j] = 0;
     }
   }

@@ -93,6 +93,23 @@ def test_repeated_centroids(gpu, s, k, dtype, pad):
         _check(x.to(dtype), gpu, k, iters=iters, seed=iters)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_many_rounds_of_small_steps(gpu, dtype):
+    """Centroids that start far out, jump to the tokens in one round and then
+    creep for hundreds: steps below the last bit of their path so far still
+    move the bounds."""
+    g = torch.Generator().manual_seed(2)
+    s, h, d, k, seed = 3000, 2, 64, 16, 9
+    x = 1e-3 * torch.randn(1, s, h, d, generator=g)
+    x[..., 0] = (torch.rand(1, s, h, generator=g) - 0.5)
+    for i in range(h):   # the initial centroids: far tokens in random directions
+        for j in range(k):
+            far = torch.randn(d, generator=g)
+            x[0, j * (s // k) + okm.mix(seed, i, k, j) % (s // k), i] = 2000.0 * far / far.norm()
+    for iters in (3, 400):
+        _check(x.to(dtype), gpu, k, iters=iters, seed=seed)
+
+
 @pytest.mark.parametrize("k,repeats", [(1, 0), (30, 0), (31, 0), (62, 0), (63, 0), (32, 1), (40, 1), (64, 2), (31, 5)])
 @pytest.mark.parametrize("norm2", [0.9e38, 2.2e38, 3.0e38])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
